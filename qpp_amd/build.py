@@ -17,6 +17,7 @@ SOURCES = [
     "qs_api.hip",
     "qs_gates.hip",
     "qs_maps.hip",
+    "qs_ptrace.hip",
     "qs_measure.hip",
     "qs_fused.hip",
     "qs_program.hip",

@@ -17,6 +17,7 @@
 
 #include <cstdint>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/qpp_amd.h"
@@ -117,6 +118,12 @@ struct QuditGate {
 };
 int launch_qudit_gate(qs_state* st, const QuditGate& g, const double* mats,
                       uint32_t nmats, uint64_t DA, bool conj);
+
+// Partial trace of a ket or density matrix into `out` (kept subsystems
+// ascending, traced ones in target order; dimension and row stride of each).
+int launch_ptrace(const qs_state* in, qs_state* out,
+                  const std::vector<std::pair<uint64_t, uint64_t>>& keep,
+                  const std::vector<std::pair<uint64_t, uint64_t>>& traced);
 
 // QEngine::execute(reps) on an engine whose gate prefix (the steps before
 // the first measurement) has already been applied elsewhere: `prefixed`

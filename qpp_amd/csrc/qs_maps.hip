@@ -1,4 +1,5 @@
-// qs_maps.hip -- ptrace, ptranspose and syspermute (out of place).
+// qs_maps.hip -- ptranspose and syspermute (out of place), and the checks of
+// ptrace (its kernels: qs_ptrace.hip).
 //
 //   k_bitperm    out[y] = in[G(y)] for a permutation G of the index bits:
 //                syspermute of qubit kets / density matrices and ptranspose
@@ -11,8 +12,6 @@
 //                from a table k_bitperm_table builds once per call.
 //   k_digitperm  the same map for qudit states (mixed-radix digits).
 //   k_ket_pt     ptranspose of a ket: out(i, j) = psi(i') conj(psi(j')).
-//   k_ptrace     partial trace; `LANES` lanes cooperate on one output entry
-//                and reduce with wavefront shuffles.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -26,17 +25,6 @@ namespace {
 
 using qs::fail;
 
-template <typename T>
-struct Real;
-template <>
-struct Real<double2> {
-    using R = double;
-};
-template <>
-struct Real<float2> {
-    using R = float;
-};
-
 // ---------------------------------------------------------------------------
 // bit-permutation gather through LDS
 // ---------------------------------------------------------------------------
@@ -48,16 +36,8 @@ struct BitPerm {
     uint8_t rest[64];      // output bits outside T, ascending
 };
 
-__device__ __forceinline__ uint64_t gather_bits(uint64_t y, const uint8_t* src,
-                                                uint32_t nb) {
-    uint64_t x = 0;
-    for (uint32_t b = 0; b < nb; ++b) x |= ((y >> b) & 1) << src[b];
-    return x;
-}
-
 // Largest tile: 2^12 elements, i.e. 16 per thread of a 256-thread workgroup.
 constexpr uint32_t kBpMaxTileBits = 12;
-constexpr int kBpPer = 1 << (kBpMaxTileBits - 8);
 
 // Every index is XOR-linear (here: OR of disjoint bits) in the element's
 // position e inside the tile and in the tile number: G and the LDS packing
@@ -208,67 +188,6 @@ __global__ __launch_bounds__(256) void k_ket_pt(const T* __restrict__ psi,
         v.x = a.x * b.x + a.y * b.y;
         v.y = a.y * b.x - a.x * b.y;
         out[y] = v;
-    }
-}
-
-// ---------------------------------------------------------------------------
-// partial trace
-// ---------------------------------------------------------------------------
-struct PT {
-    uint32_t nkeep, ntr;
-    uint64_t kdim[40], kstr[40];  // kept subsystems (ascending), row strides
-    uint64_t tdim[40], tstr[40];  // traced subsystems (target order)
-    uint64_t Dbar, Dsub, D;
-    uint32_t rho;
-};
-
-__device__ __forceinline__ uint64_t mixed(uint64_t v, uint32_t n,
-                                          const uint64_t* dim,
-                                          const uint64_t* str) {
-    uint64_t off = 0;
-    for (int k = int(n) - 1; k >= 0; --k) {
-        off += (v % dim[k]) * str[k];
-        v /= dim[k];
-    }
-    return off;
-}
-
-template <typename T, int LANES>
-__global__ __launch_bounds__(256) void k_ptrace(const T* __restrict__ a,
-                                                T* __restrict__ out, PT p) {
-    using R = typename Real<T>::R;
-    const uint64_t groups = uint64_t(gridDim.x) * (256 / LANES);
-    const uint32_t lane = threadIdx.x % LANES;
-    const uint64_t total = p.Dbar * p.Dbar;
-    for (uint64_t o = uint64_t(blockIdx.x) * (256 / LANES) + threadIdx.x / LANES;
-         o < total + 0 * groups; o += groups) {
-        const uint64_t i = o % p.Dbar, j = o / p.Dbar;
-        const uint64_t rb = mixed(i, p.nkeep, p.kdim, p.kstr);
-        const uint64_t cb = mixed(j, p.nkeep, p.kdim, p.kstr);
-        R sr = 0, si = 0;
-        for (uint64_t t = lane; t < p.Dsub; t += LANES) {
-            const uint64_t off = mixed(t, p.ntr, p.tdim, p.tstr);
-            if (p.rho) {
-                const T v = a[(rb + off) + (cb + off) * p.D];
-                sr += v.x;
-                si += v.y;
-            } else {
-                const T x = a[rb + off], y = a[cb + off];
-                // x * conj(y)
-                sr += x.x * y.x + x.y * y.y;
-                si += x.y * y.x - x.x * y.y;
-            }
-        }
-        for (int m = LANES / 2; m > 0; m >>= 1) {
-            sr += __shfl_xor(sr, m, LANES);
-            si += __shfl_xor(si, m, LANES);
-        }
-        if (lane == 0) {
-            T v;
-            v.x = sr;
-            v.y = si;
-            out[o] = v;
-        }
     }
 }
 
@@ -443,26 +362,6 @@ int launch_ket_pt(const qs_state* in, qs_state* out, const KetPT& p) {
     return QS_OK;
 }
 
-template <typename T>
-int launch_ptrace(const qs_state* in, qs_state* out, const PT& p) {
-    const uint64_t total = p.Dbar * p.Dbar;
-    if (p.Dsub >= 64) {
-        hipLaunchKernelGGL((k_ptrace<T, 64>), dim3(grid_for(total, 4)), dim3(256), 0,
-                           in->stream, static_cast<const T*>(in->d),
-                           static_cast<T*>(out->d), p);
-    } else if (p.Dsub >= 8) {
-        hipLaunchKernelGGL((k_ptrace<T, 8>), dim3(grid_for(total, 32)), dim3(256), 0,
-                           in->stream, static_cast<const T*>(in->d),
-                           static_cast<T*>(out->d), p);
-    } else {
-        hipLaunchKernelGGL((k_ptrace<T, 1>), dim3(grid_for(total, 256)), dim3(256), 0,
-                           in->stream, static_cast<const T*>(in->d),
-                           static_cast<T*>(out->d), p);
-    }
-    QS_HIP(hipGetLastError(), "qpp::ptrace()");
-    return QS_OK;
-}
-
 }  // namespace
 
 extern "C" {
@@ -481,30 +380,15 @@ int qs_ptrace(const qs_state* st, uint32_t ntarget, const uint64_t* target,
     std::vector<uint64_t> keep;
     for (uint64_t q = 0; q < n; ++q)
         if (std::find(tv.begin(), tv.end(), q) == tv.end()) keep.push_back(q);
-    PT p{};
-    p.rho = st->kind == QS_RHO;
-    p.D = st->D;
-    p.Dbar = 1;
-    p.Dsub = 1;
-    p.nkeep = static_cast<uint32_t>(keep.size());
-    p.ntr = static_cast<uint32_t>(tv.size());
-    if (p.nkeep > 40 || p.ntr > 40) return fail(QS_ERR_NOT_IMPLEMENTED, W, "subsystems");
-    for (size_t k = 0; k < keep.size(); ++k) {
-        p.kdim[k] = st->dims[keep[k]];
-        p.kstr[k] = row_stride(st, keep[k]);
-        p.Dbar *= p.kdim[k];
-    }
-    for (size_t k = 0; k < tv.size(); ++k) {
-        p.tdim[k] = st->dims[tv[k]];
-        p.tstr[k] = row_stride(st, tv[k]);
-        p.Dsub *= p.tdim[k];
-    }
+    if (keep.size() > 40 || tv.size() > 40) return fail(QS_ERR_NOT_IMPLEMENTED, W, "subsystems");
+    std::vector<std::pair<uint64_t, uint64_t>> kd, td;  // (dimension, row stride)
+    for (uint64_t q : keep) kd.emplace_back(st->dims[q], row_stride(st, q));
+    for (uint64_t q : tv) td.emplace_back(st->dims[q], row_stride(st, q));
     std::vector<uint64_t> odims;
     for (uint64_t q : keep) odims.push_back(st->dims[q]);
     if (odims.empty()) odims.push_back(1);  // full trace: a 1 x 1 matrix
     if (int rc = make_out(st, QS_RHO, odims, out)) return rc;
-    return st->dtype == QS_C128 ? launch_ptrace<double2>(st, *out, p)
-                                : launch_ptrace<float2>(st, *out, p);
+    return qs::launch_ptrace(st, *out, kd, td);
 }
 
 // qpp::ptranspose(A, target, dims), operations.hpp:2167-2335 (documented);
