@@ -565,8 +565,9 @@ def bench_block(args, qa, n=30, reps=3):
     """Dense 4- and 5-qubit gates (16x16 and 32x32 unitaries, the widest
     blocks qpp::apply takes on the matrix cores here) on an n-qubit
     complex64 ket, every amplitude read and written once per launch: the
-    FP32 MFMA kernel (k_gatek_mfma) against the VALU kernel (k_gatek, forced
-    with QPP_AMD_GATEK_VALU=1), plus the complex128 VALU kernel.  HBM
+    kernels that take them (k_gate_reg for 4 qubits, the FP32 MFMA kernel
+    k_gatek_mfma for 5) against the kernel for any width (k_gatek, forced
+    with QPP_AMD_GATEK_VALU=1), plus complex128 (k_gate_reg, k_gatek).  HBM
     roofline: 2 s 2^n bytes per launch; arithmetic: 4 x 2^k real FMA per
     amplitude on either unit (the complex product as a real GEMM)."""
     import os
@@ -577,8 +578,8 @@ def bench_block(args, qa, n=30, reps=3):
         U = haar(2 ** k, rng)
         tg = [0, 7, 13, 21, 29][:k]  # low and high target bits
         row = {"qubits_in_gate": k, "targets": tg}
-        for label, dt, valu in (("c64_mfma", qa.C64, False), ("c64_valu", qa.C64, True),
-                                ("c128_valu", qa.C128, True)):
+        for label, dt, valu in (("c64", qa.C64, False), ("c64_valu", qa.C64, True),
+                                ("c128", qa.C128, False)):
             st = qa.State([2] * n, dtype=dt)
             if valu:
                 os.environ["QPP_AMD_GATEK_VALU"] = "1"
@@ -595,13 +596,15 @@ def bench_block(args, qa, n=30, reps=3):
                           "hbm_frac": round(gbs / HBM_PEAK_GBS, 4),
                           "TFLOPs": round(fl / (ms / 1e3) / 1e12, 2)}
             del st
-        row["c64_mfma"]["mfma_frac"] = round(row["c64_mfma"]["TFLOPs"] / 157.3, 4)
-        row["mfma_speedup_vs_valu"] = round(row["c64_valu"]["ms"] / row["c64_mfma"]["ms"], 3)
+        row["c64"]["kernel"] = "k_gate_reg<float,4>" if k == 4 else "k_gatek_mfma<5>"
+        if k == 5:
+            row["c64"]["mfma_frac"] = round(row["c64"]["TFLOPs"] / 157.3, 4)
+        row["speedup_vs_valu"] = round(row["c64_valu"]["ms"] / row["c64"]["ms"], 3)
         log(f"block k={k}: {row}")
         out.append(row)
     # the 5-qubit gate is the MFMA-heavy case: its roofline against the FP32
     # matrix peak, beside its HBM rate
-    k5 = out[-1]["c64_mfma"]
+    k5 = out[-1]["c64"]
     roof = {"bound": "mfma", "kernel": "k_gatek_mfma<5>", "achieved": k5["TFLOPs"], "peak": 157.3,
             "unit": "TFLOP/s", "frac": round(k5["TFLOPs"] / 157.3, 4), "traffic": None,
             "avg_launch_ms": k5["ms"], "hbm_GBps": k5["GBps"], "hbm_frac": k5["hbm_frac"]}

@@ -244,21 +244,26 @@ int gate_dispatch(qs_state* st, const double* A, uint64_t dimA,
     const bool rho = st->kind == QS_RHO;
     if (st->qubits) {
         const uint32_t k = static_cast<uint32_t>(target.size());
-        for (int pass = 0; pass < (rho ? 2 : 1); ++pass) {
-            const bool cols = pass == 1;
-            std::vector<uint32_t> bits(k);
-            for (uint32_t i = 0; i < k; ++i)
-                bits[i] = cols ? col_bit(st, target[i]) : row_bit(st, target[i]);
-            uint64_t cmask = 0, cval = 0;
+        // bits of the targets and masks of the controls on the rows, then (for
+        // a density matrix) the columns
+        std::vector<uint32_t> bits[2];
+        uint64_t cmask[2] = {0, 0}, cval[2] = {0, 0};
+        for (int cols = 0; cols < (rho ? 2 : 1); ++cols) {
+            for (uint64_t t : target) bits[cols].push_back(cols ? col_bit(st, t) : row_bit(st, t));
             for (size_t c = 0; c < ctrl.size(); ++c) {
                 const uint32_t b = cols ? col_bit(st, ctrl[c]) : row_bit(st, ctrl[c]);
-                cmask |= uint64_t{1} << b;
+                cmask[cols] |= uint64_t{1} << b;
                 // shift 0: control on |1>, shift 1: on |0> (apply_ctrl.hpp:123-132)
-                if (shift[c] == 0) cval |= uint64_t{1} << b;
+                if (shift[c] == 0) cval[cols] |= uint64_t{1} << b;
             }
-            if (int rc = qs::launch_gatek(st, bits.data(), k, A, cmask, cval, cols))
-                return rc;
         }
+        if (rho && k <= 2) {
+            bits[1].insert(bits[1].end(), bits[0].begin(), bits[0].end());
+            return qs::launch_gate_rho(st, bits[1].data(), k, A, cmask, cval);
+        }
+        for (int cols = 0; cols < (rho ? 2 : 1); ++cols)
+            if (int rc = qs::launch_gatek(st, bits[cols].data(), k, A, cmask[cols], cval[cols], cols))
+                return rc;
         return QS_OK;
     }
     // qudits: A^r table for controlled gates (operations.hpp:777-782)
@@ -408,6 +413,7 @@ int qs_state_create(qs_dtype dtype, qs_kind kind, uint32_t ndims,
 int qs_state_destroy(qs_state* st) {
     if (!st) return QS_OK;
     if (st->d) (void)hipFreeAsync(st->d, st->stream);
+    if (st->tab) (void)hipFreeAsync(st->tab, st->stream);
     delete st;
     return QS_OK;
 }

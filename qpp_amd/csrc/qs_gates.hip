@@ -12,11 +12,13 @@
 //               the same 64-element aligned chunk, i.e. in another lane of
 //               the same wave; lanes load consecutive elements (fully
 //               coalesced) and exchange partners with a lane shuffle.
-//   k_gatek     k-bit dense gate (k <= 10) through LDS: a workgroup stages a
+//   k_gate_reg  2- to 4-bit dense gates (complex64: 2 and 3 bits), and 1- and
+//               2-qubit gates on both sides of a density matrix in one pass:
+//               a thread's group of amplitudes in registers.
+//   k_gatek     wider dense gates (k <= 10) through LDS: a workgroup stages a
 //               batch of amplitude groups, each thread then forms outputs
 //               from the staged group and the gate matrix.
-//   k_gatek_mfma  4- and 5-bit dense gates on complex64 states with FP32
-//               MFMA: Y = U X over the state's amplitude groups as a real
+//   k_gatek_mfma  5-bit dense gates on complex64 states with FP32 MFMA: Y = U X over the state's amplitude groups as a real
 //               GEMM (2^(k+1) x 2^(k+1) times 16 groups per wave step).
 //   k_qudit     mixed-radix gate for qudit states (multi-index strides).
 //
@@ -52,6 +54,12 @@ __device__ __forceinline__ cxt<R> cmul(cxt<R> a, cxt<R> b) {
     r.x = a.x * b.x - a.y * b.y;
     r.y = a.x * b.y + a.y * b.x;
     return r;
+}
+
+template <typename R>
+__device__ __forceinline__ cxt<R> conj_c(cxt<R> a) {
+    a.y = -a.y;
+    return a;
 }
 
 template <typename R>
@@ -188,6 +196,146 @@ __global__ __launch_bounds__(kBlock) void k_gate1_lo(cxt<R>* __restrict__ a,
 }
 
 // ---------------------------------------------------------------------------
+// 2- to 4-bit dense gates in registers
+// ---------------------------------------------------------------------------
+// A thread holds the 2^K amplitudes of one group in registers, multiplies
+// them by the gate and stores them; HBM bounds it (16 FP64 FMA per amplitude
+// at K = 2, 64 at K = 4, against 32 bytes).  Every load and store runs over
+// 64 consecutive amplitudes: a target bit below 6 is one of the lane bits
+// there, so its place among the register bits is taken by the lowest free
+// bit above, and after the loads the two are exchanged (half of the
+// registers with the lane across that bit), and back before the stores.
+// Loading the groups of a low target directly instead would touch every
+// line 2^K times.
+//
+// RHO: a density matrix's U rho U^dagger in one pass: the register bits are
+// the K/2 column targets, then the K/2 row targets; U goes to the row bits
+// where the row controls hold and conj(U) to the column bits where the
+// column controls hold.  11 qubits complex128: 37 -> 18 us for one qubit (two
+// passes before), 94-125 -> 20 us for two.
+struct RegGate {
+    Fixed fx;            // squeezed out of the group index: register bits, high controls
+    uint64_t cval;       // the high controls' values
+    uint64_t off[16];    // offset of register c (before the exchange)
+    uint64_t mask[2], val[2];  // RHO: row and column controls; else mask[0]: low controls
+    int8_t lane_bit[4];  // lane bit to exchange with register bit j, or -1
+};
+
+template <typename R, int DIM, bool BYVAL>
+struct GateMat {
+    cxt<R> m[DIM * DIM];
+    __device__ __forceinline__ cxt<R> at(int i) const { return m[i]; }
+};
+template <typename R, int DIM>
+struct GateMat<R, DIM, false> {
+    const cxt<R>* m;
+    __device__ __forceinline__ cxt<R> at(int i) const { return m[i]; }
+};
+// a matrix of up to 1 KiB travels in the kernel's arguments
+template <typename R, int K, bool RHO>
+using RegMat = GateMat<R, RHO ? (1 << (K / 2)) : (1 << K), RHO || K <= 3>;
+
+template <typename R, int K>
+__device__ __forceinline__ void exchange(cxt<R> (&x)[1 << K], const int8_t (&lane_bit)[4]) {
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        const int b = lane_bit[j];
+        if (b < 0) continue;
+        const bool one = (threadIdx.x >> b) & 1;
+#pragma unroll
+        for (int c = 0; c < (1 << K); ++c) {
+            if ((c >> j) & 1) continue;
+            const cxt<R> lo = x[c], hi = x[c | (1 << j)];
+            cxt<R> give;
+            give.x = one ? lo.x : hi.x;
+            give.y = one ? lo.y : hi.y;
+            const cxt<R> got = shfl_xor_c<R>(give, 1 << b);
+            x[c].x = one ? got.x : lo.x;
+            x[c].y = one ? got.y : lo.y;
+            x[c | (1 << j)].x = one ? hi.x : got.x;
+            x[c | (1 << j)].y = one ? hi.y : got.y;
+        }
+    }
+}
+
+template <typename R, int K, bool RHO, int NG>
+__global__ __launch_bounds__(kBlock) void k_gate_reg(cxt<R>* __restrict__ a, uint64_t ngroups, RegGate g,
+                                                     RegMat<R, K, RHO> m) {
+    constexpr int DIM = 1 << K;
+    const uint64_t nthreads = uint64_t(gridDim.x) * kBlock;
+    const uint64_t p = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
+    cxt<R> x[NG][DIM];
+    uint64_t base[NG];
+    bool act[NG], rows[NG], cols[NG];
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+        const uint64_t q = p + i * nthreads;
+        base[i] = insert_zeros(q, g.fx.pos, g.fx.np) | g.cval;
+        rows[i] = (base[i] & g.mask[0]) == g.val[0];
+        cols[i] = RHO && (base[i] & g.mask[1]) == g.val[1];
+        act[i] = q < ngroups && (rows[i] || cols[i]);
+#pragma unroll
+        for (int c = 0; c < DIM; ++c) {
+            x[i][c].x = 0;
+            x[i][c].y = 0;
+            if (act[i]) x[i][c] = a[base[i] + g.off[c]];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NG; ++i) {
+        // (a lane and those it exchanges with have the same controls)
+        exchange<R, K>(x[i], g.lane_bit);
+        if constexpr (RHO) {
+            constexpr int D = 1 << (K / 2);
+            if (rows[i]) {
+#pragma unroll
+                for (int h = 0; h < D; ++h) {
+                    cxt<R> in[D];
+#pragma unroll
+                    for (int c = 0; c < D; ++c) in[c] = x[i][h * D + c];
+#pragma unroll
+                    for (int r = 0; r < D; ++r) {
+                        cxt<R> acc = cmul<R>(m.at(r), in[0]);
+#pragma unroll
+                        for (int c = 1; c < D; ++c) acc = cfma<R>(m.at(r + c * D), in[c], acc);
+                        x[i][h * D + r] = acc;
+                    }
+                }
+            }
+            if (cols[i]) {
+#pragma unroll
+                for (int h = 0; h < D; ++h) {
+                    cxt<R> in[D];
+#pragma unroll
+                    for (int c = 0; c < D; ++c) in[c] = x[i][c * D + h];
+#pragma unroll
+                    for (int r = 0; r < D; ++r) {
+                        cxt<R> acc = cmul<R>(conj_c<R>(m.at(r)), in[0]);
+#pragma unroll
+                        for (int c = 1; c < D; ++c) acc = cfma<R>(conj_c<R>(m.at(r + c * D)), in[c], acc);
+                        x[i][r * D + h] = acc;
+                    }
+                }
+            }
+        } else {
+            cxt<R> y[DIM];
+#pragma unroll
+            for (int r = 0; r < DIM; ++r) y[r] = cmul<R>(m.at(r), x[i][0]);
+#pragma unroll
+            for (int c = 1; c < DIM; ++c)
+#pragma unroll
+                for (int r = 0; r < DIM; ++r) y[r] = cfma<R>(m.at(r + c * DIM), x[i][c], y[r]);
+#pragma unroll
+            for (int r = 0; r < DIM; ++r) x[i][r] = y[r];
+        }
+        exchange<R, K>(x[i], g.lane_bit);
+#pragma unroll
+        for (int c = 0; c < DIM; ++c)
+            if (act[i]) a[base[i] + g.off[c]] = x[i][c];
+    }
+}
+
+// ---------------------------------------------------------------------------
 // k-bit dense gate through LDS
 // ---------------------------------------------------------------------------
 // Groups: the 2^k elements sharing all non-target bits.  The group index g
@@ -237,7 +385,7 @@ __global__ __launch_bounds__(kBlock) void k_gatek(
 }
 
 // ---------------------------------------------------------------------------
-// k-bit dense gate with MFMA (complex64, k = 4, 5)
+// 5-bit dense gate with MFMA (complex64)
 // ---------------------------------------------------------------------------
 // The groups (columns) are as in k_gatek.  Over the real and imaginary parts
 // the gate is one real GEMM, [Yr; Yi] = W [Xr; Xi] with W = [[Ur, -Ui],
@@ -348,75 +496,28 @@ __global__ __launch_bounds__(kBlock) void k_gatek_mfma(float2* __restrict__ a, u
     // group again (in bounds, never used): with no load under a branch the
     // waits before each group's products count exactly the loads and
     // stores issued after its own loads
-    if constexpr (K == 4) {
-        // 4 amplitudes per lane and group, 8 waves per SIMD: the next group
-        // in flight, loaded under the lanes' bounds and copied into place
-        float yr[NX], yi[NX];
-        Buf cur;
-        cur.ok = false;
-        bool ok = (grp * 16 + j) < ncols;
-        uint64_t base = ok ? (insert_zeros(grp * 16 + j, fx.pos, fx.np) | cval) : 0;
-#pragma unroll
-        for (int q = 0; q < NX; ++q) {
-            float2 v = make_float2(0.f, 0.f);
-            if (ok) v = a[base + in_off[q]];
-            cur.xr[q] = v.x;
-            cur.xi[q] = v.y;
-        }
-        for (;;) {
-            const uint64_t next = grp + nwaves;
-            const bool more = next * 16 < ncols;  // uniform over the wave
-            uint64_t nbase = 0;
-            bool nok = false;
-            if (more) {
-                const uint64_t col = next * 16 + j;
-                nok = col < ncols;
-                nbase = nok ? (insert_zeros(col, fx.pos, fx.np) | cval) : 0;
-#pragma unroll
-                for (int q = 0; q < NX; ++q) {
-                    float2 v = make_float2(0.f, 0.f);
-                    if (nok) v = a[nbase + in_off[q]];
-                    yr[q] = v.x;
-                    yi[q] = v.y;
-                }
-            }
-            cur.base = base;
-            cur.ok = ok;
-            process(cur);
-            if (!more) break;
-            grp = next;
-            base = nbase;
-            ok = nok;
-#pragma unroll
-            for (int q = 0; q < NX; ++q) {
-                cur.xr[q] = yr[q];
-                cur.xi[q] = yi[q];
-            }
-        }
-    } else {
-        // 8 amplitudes per lane and group, 4 waves per SIMD: the next two
-        // groups in flight (three buffers in turn)
-        Buf b0, b1, b2;
-        fetch(grp, b0);
-        bool has1 = (grp + nwaves) * 16 < ncols;
-        fetch(has1 ? grp + nwaves : grp, b1);
-        // `cur` holds group grp, the next buffer group grp + nwaves (when
-        // has1), and `far` receives group grp + 2 nwaves; false once grp was
-        // the last
-        auto step = [&](const Buf& cur, Buf& far) {
-            const bool has2 = (grp + 2 * nwaves) * 16 < ncols;
-            fetch(has2 ? grp + 2 * nwaves : grp, far);
-            process(cur);
-            if (!has1) return false;
-            grp += nwaves;
-            has1 = has2;
-            return true;
-        };
-        for (;;) {
-            if (!step(b0, b2)) break;
-            if (!step(b1, b0)) break;
-            if (!step(b2, b1)) break;
-        }
+    // 8 amplitudes per lane and group, 4 waves per SIMD: the next two
+    // groups in flight (three buffers in turn)
+    Buf b0, b1, b2;
+    fetch(grp, b0);
+    bool has1 = (grp + nwaves) * 16 < ncols;
+    fetch(has1 ? grp + nwaves : grp, b1);
+    // `cur` holds group grp, the next buffer group grp + nwaves (when
+    // has1), and `far` receives group grp + 2 nwaves; false once grp was
+    // the last
+    auto step = [&](const Buf& cur, Buf& far) {
+        const bool has2 = (grp + 2 * nwaves) * 16 < ncols;
+        fetch(has2 ? grp + 2 * nwaves : grp, far);
+        process(cur);
+        if (!has1) return false;
+        grp += nwaves;
+        has1 = has2;
+        return true;
+    };
+    for (;;) {
+        if (!step(b0, b2)) break;
+        if (!step(b1, b0)) break;
+        if (!step(b2, b1)) break;
     }
 }
 
@@ -543,21 +644,124 @@ int gate1_impl(qs_state* st, uint32_t bit, const double* m, uint64_t cmask,
     return QS_OK;
 }
 
-// Device scratch for gate matrices / index tables of one call.  Kept per
-// state so stream ordering on the state's stream protects reuse.
-struct Scratch {
-    void* d = nullptr;
-    size_t bytes = 0;
+// Up to 3 KiB of a host table, carried in a kernel's arguments to device
+// memory: ordered on the stream without the host waiting for a copy.
+struct PutChunk {
+    uint32_t w[768];
 };
+__global__ __launch_bounds__(256) void k_put(uint32_t* __restrict__ d, PutChunk c, uint32_t n) {
+    for (uint32_t i = threadIdx.x; i < n; i += 256) d[i] = c.w[i];
+}
 
-int upload(qs_state* st, const void* host, size_t bytes, void** dptr) {
-    // one allocation per call, freed stream-ordered after the kernel
-    QS_HIP(hipMallocAsync(dptr, bytes, st->stream), "qpp_amd::upload");
-    QS_HIP(hipMemcpyAsync(*dptr, host, bytes, hipMemcpyHostToDevice, st->stream),
-           "qpp_amd::upload");
+// Device copy of a host table of one call (matrices, offsets), a multiple of
+// 4 bytes.  Up to kTabBytes it goes into the state's own table memory, which
+// its next call overwrites in stream order: a few launches, where an
+// allocation, a pageable copy, its wait and the free took 25 us (16 KiB: six
+// launches).  Larger tables are copied into memory of their own (*owned),
+// freed stream-ordered after the kernel.
+constexpr size_t kTabBytes = 24576;
+
+int upload(qs_state* st, const void* host, size_t bytes, void** dptr, void** owned) {
+    constexpr const char* W = "qpp_amd::upload";
+    *owned = nullptr;
+    if (bytes <= kTabBytes) {
+        if (!st->tab) QS_HIP(hipMallocAsync(&st->tab, kTabBytes, st->stream), W);
+        *dptr = st->tab;
+        PutChunk c;
+        for (size_t at = 0; at < bytes; at += sizeof(c)) {
+            const size_t part = std::min(sizeof(c), bytes - at);
+            std::memcpy(c.w, static_cast<const char*>(host) + at, part);
+            hipLaunchKernelGGL(k_put, dim3(1), dim3(256), 0, st->stream,
+                               reinterpret_cast<uint32_t*>(static_cast<char*>(st->tab) + at), c,
+                               static_cast<uint32_t>(part / 4));
+        }
+        QS_HIP(hipGetLastError(), W);
+        return QS_OK;
+    }
+    QS_HIP(hipMallocAsync(owned, bytes, st->stream), W);
+    *dptr = *owned;
+    hipError_t e = hipMemcpyAsync(*owned, host, bytes, hipMemcpyHostToDevice, st->stream);
     // pageable source: make sure the copy has consumed `host` before return
-    QS_HIP(hipStreamSynchronize(st->stream), "qpp_amd::upload");
+    if (e == hipSuccess) e = hipStreamSynchronize(st->stream);
+    if (e != hipSuccess) {
+        (void)hipFreeAsync(*owned, st->stream);
+        return qs::fail_hip(e, W);
+    }
     return QS_OK;
+}
+
+// Descriptor of k_gate_reg: `regs` the bits of register bits K-1 .. 0, the
+// controls as masks of the index (RHO: rows then columns).
+RegGate reg_gate(uint32_t nb, const uint32_t* regs, uint32_t K, bool rho, const uint64_t (&cmask)[2],
+                 const uint64_t (&cval)[2], uint64_t* ngroups) {
+    RegGate g{};
+    const uint64_t ctrl = cmask[0] | cmask[1];
+    uint64_t used = ctrl;
+    uint32_t low = 0;
+    for (uint32_t j = 0; j < K; ++j) {
+        used |= uint64_t{1} << regs[j];
+        low += regs[j] < 6;
+    }
+    std::vector<uint32_t> free_bits;
+    for (uint32_t b = 6; b < nb && free_bits.size() < low; ++b)
+        if (!((used >> b) & 1)) free_bits.push_back(b);
+    // a register too small for whole waves of groups takes one group a lane
+    // with the targets where they are
+    const bool lanes = free_bits.size() == low && nb >= 6;
+    const uint64_t squeezed = rho ? 0 : lanes ? ctrl & ~uint64_t{63} : ctrl;
+    std::vector<uint32_t> fixed = bits_of(squeezed);
+    uint32_t next = 0;
+    for (uint32_t j = 0; j < 4; ++j) g.lane_bit[j] = -1;
+    uint64_t bit_off[4] = {};
+    for (uint32_t j = 0; j < K; ++j) {
+        uint32_t b = regs[K - 1 - j];  // register bit j
+        if (lanes && b < 6) {
+            g.lane_bit[j] = static_cast<int8_t>(b);
+            b = free_bits[next++];
+        }
+        fixed.push_back(b);
+        bit_off[j] = uint64_t{1} << b;
+    }
+    for (uint32_t c = 0; c < (1u << K); ++c)
+        for (uint32_t j = 0; j < K; ++j)
+            if ((c >> j) & 1) g.off[c] |= bit_off[j];
+    g.fx = make_fixed(fixed);
+    g.cval = cval[0] & squeezed;
+    for (int i = 0; i < 2; ++i) {
+        g.mask[i] = cmask[i] & ~squeezed;
+        g.val[i] = cval[i] & g.mask[i];
+    }
+    *ngroups = uint64_t{1} << (nb - g.fx.np);
+    return g;
+}
+
+template <typename R, int K, bool RHO>
+int gate_reg(qs_state* st, const uint32_t* regs, const double* m, bool conj, const uint64_t (&cmask)[2],
+             const uint64_t (&cval)[2]) {
+    constexpr int DIM = RHO ? 1 << (K / 2) : 1 << K;
+    uint64_t ngroups = 0;
+    const RegGate g = reg_gate(st->nbits, regs, K, RHO, cmask, cval, &ngroups);
+    // small groups: 128 bytes of loads in flight per thread
+    constexpr int NG = K >= 4 ? 1 : (sizeof(R) == 8 ? 8 : 16) >> K;
+    const uint32_t grid = grid_for(ngroups, uint64_t(kBlock) * NG);
+    auto* a = static_cast<cxt<R>*>(st->d);
+    RegMat<R, K, RHO> mat;
+    if constexpr (RHO || K <= 3) {
+        for (int i = 0; i < DIM * DIM; ++i) mat.m[i] = to_c<R>(m, i, conj);
+        hipLaunchKernelGGL((k_gate_reg<R, K, RHO, NG>), dim3(grid), dim3(kBlock), 0, st->stream, a, ngroups, g,
+                           mat);
+        return QS_OK;
+    } else {
+        cxt<R> mm[DIM * DIM];
+        for (int i = 0; i < DIM * DIM; ++i) mm[i] = to_c<R>(m, i, conj);
+        void *d = nullptr, *owned = nullptr;
+        static_assert(sizeof(mm) <= kTabBytes, "in the state's table memory");
+        if (int rc = upload(st, mm, sizeof(mm), &d, &owned)) return rc;
+        mat.m = static_cast<const cxt<R>*>(d);
+        hipLaunchKernelGGL((k_gate_reg<R, K, RHO, NG>), dim3(grid), dim3(kBlock), 0, st->stream, a, ngroups, g,
+                           mat);
+        return QS_OK;
+    }
 }
 
 int gatek_mfma(qs_state* st, uint32_t k, const std::vector<uint64_t>& inner, const double* m,
@@ -566,6 +770,11 @@ int gatek_mfma(qs_state* st, uint32_t k, const std::vector<uint64_t>& inner, con
 template <typename R>
 int gatek_impl(qs_state* st, const uint32_t* bits, uint32_t k, const double* m,
                uint64_t cmask, uint64_t cval, bool conj) {
+    constexpr bool f64 = std::is_same<R, double>::value;
+    const uint64_t cm[2] = {cmask, 0}, cv[2] = {cval, 0};
+    if (k == 2) return gate_reg<R, 2, false>(st, bits, m, conj, cm, cv);
+    if (k == 3) return gate_reg<R, 3, false>(st, bits, m, conj, cm, cv);
+    if (k == 4 && (f64 || !qs::gatek_valu_forced())) return gate_reg<R, 4, false>(st, bits, m, conj, cm, cv);
     const uint32_t dim = 1u << k;
     std::vector<uint64_t> inner(dim);
     for (uint32_t c = 0; c < dim; ++c) {
@@ -581,16 +790,16 @@ int gatek_impl(qs_state* st, const uint32_t* bits, uint32_t k, const double* m,
     for (uint32_t b : bits_of(cmask)) fixed.push_back(b);
     const Fixed fx = make_fixed(fixed);
     const uint64_t ngroups = uint64_t{1} << (st->nbits - fx.np);
-    if constexpr (std::is_same<R, float>::value)
-        if ((k == 4 || k == 5) && !qs::gatek_valu_forced())
+    if constexpr (!f64)
+        if (k == 5 && !qs::gatek_valu_forced())
             return gatek_mfma(st, k, inner, m, conj, fx, cval, ngroups);
     const size_t inner_bytes = inner.size() * sizeof(uint64_t);
     const size_t mat_bytes = mm.size() * sizeof(cxt<R>);
     std::vector<unsigned char> blob(inner_bytes + mat_bytes);
     std::memcpy(blob.data(), inner.data(), inner_bytes);
     std::memcpy(blob.data() + inner_bytes, mm.data(), mat_bytes);
-    void* dblob = nullptr;
-    if (int rc = upload(st, blob.data(), blob.size(), &dblob)) return rc;
+    void *dblob = nullptr, *owned = nullptr;
+    if (int rc = upload(st, blob.data(), blob.size(), &dblob, &owned)) return rc;
     constexpr int EPT = 4;
     // groups per block must be >= 1: for dim > kBlock*EPT use larger EPT
     int G = (kBlock * EPT) >> k;
@@ -604,7 +813,7 @@ int gatek_impl(qs_state* st, const uint32_t* bits, uint32_t k, const double* m,
                        reinterpret_cast<const cxt<R>*>(
                            static_cast<unsigned char*>(dblob) + inner_bytes),
                        fx, cval, uint64_t{0}, uint64_t{0});
-    QS_HIP(hipFreeAsync(dblob, st->stream), "qpp_amd::apply");
+    if (owned) QS_HIP(hipFreeAsync(owned, st->stream), "qpp_amd::apply");
     return QS_OK;
 }
 
@@ -633,25 +842,21 @@ int gatek_mfma(qs_state* st, uint32_t k, const std::vector<uint64_t>& inner, con
     // more workgroups than are resident at once, so none starts late
     const uint64_t groups16 = (ncols + 15) / 16;
     int per_cu = 0, dev = 0, ncu = 0;
-    QS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k == 4 ? k_gatek_mfma<4> : k_gatek_mfma<5>,
+    QS_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_gatek_mfma<5>,
                                                         kBlock, 0),
            "qpp::apply()");
     QS_HIP(hipGetDevice(&dev), "qpp::apply()");
     QS_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "qpp::apply()");
     const uint32_t resident = static_cast<uint32_t>(std::max(1, per_cu) * std::max(1, ncu));
     const uint32_t grid = std::min<uint32_t>(grid_for(groups16, kBlock / 64), std::min(kMfmaGrid, resident));
-    void* dblob = nullptr;
-    if (int rc = upload(st, blob.data(), blob.size(), &dblob)) return rc;
+    void *dblob = nullptr, *owned = nullptr;
+    if (int rc = upload(st, blob.data(), blob.size(), &dblob, &owned)) return rc;
     auto* inn = static_cast<const uint64_t*>(dblob);
     auto* wpk = reinterpret_cast<const float*>(static_cast<unsigned char*>(dblob) + inner_bytes);
-    if (k == 4)
-        hipLaunchKernelGGL(k_gatek_mfma<4>, dim3(grid), dim3(kBlock), 0, st->stream,
-                           static_cast<float2*>(st->d), ncols, inn, wpk, fx, cval);
-    else
-        hipLaunchKernelGGL(k_gatek_mfma<5>, dim3(grid), dim3(kBlock), 0, st->stream,
-                           static_cast<float2*>(st->d), ncols, inn, wpk, fx, cval);
+    hipLaunchKernelGGL(k_gatek_mfma<5>, dim3(grid), dim3(kBlock), 0, st->stream,
+                       static_cast<float2*>(st->d), ncols, inn, wpk, fx, cval);
     QS_HIP(hipGetLastError(), "qpp::apply()");
-    QS_HIP(hipFreeAsync(dblob, st->stream), "qpp_amd::apply");
+    if (owned) QS_HIP(hipFreeAsync(owned, st->stream), "qpp_amd::apply");
     return QS_OK;
 }
 
@@ -694,15 +899,15 @@ int qudit_impl(qs_state* st, const qs::QuditGate& g, const double* mats,
     std::vector<unsigned char> blob(off_bytes + mat_bytes);
     std::memcpy(blob.data(), off.data(), off_bytes);
     std::memcpy(blob.data() + off_bytes, mm.data(), mat_bytes);
-    void* dblob = nullptr;
-    if (int rc = upload(st, blob.data(), blob.size(), &dblob)) return rc;
+    void *dblob = nullptr, *owned = nullptr;
+    if (int rc = upload(st, blob.data(), blob.size(), &dblob, &owned)) return rc;
     const uint32_t grid = grid_for(nspec, kBlock);
     hipLaunchKernelGGL((k_qudit<R>), dim3(grid), dim3(kBlock), 0, st->stream,
                        static_cast<cxt<R>*>(st->d), nspec, q,
                        reinterpret_cast<const cxt<R>*>(
                            static_cast<unsigned char*>(dblob) + off_bytes),
                        static_cast<const uint64_t*>(dblob));
-    QS_HIP(hipFreeAsync(dblob, st->stream), "qpp_amd::apply");
+    if (owned) QS_HIP(hipFreeAsync(owned, st->stream), "qpp_amd::apply");
     return QS_OK;
 }
 
@@ -726,6 +931,20 @@ int launch_gatek(qs_state* st, const uint32_t* bits, uint32_t k,
     int rc = st->dtype == QS_C128
                  ? gatek_impl<double>(st, bits, k, m, cmask, cval, conj)
                  : gatek_impl<float>(st, bits, k, m, cmask, cval, conj);
+    if (rc) return rc;
+    QS_HIP(hipGetLastError(), "qpp::apply()");
+    return QS_OK;
+}
+
+int launch_gate_rho(qs_state* st, const uint32_t* bits, uint32_t k, const double* m,
+                    const uint64_t (&cmask)[2], const uint64_t (&cval)[2]) {
+    int rc = QS_OK;
+    if (k == 1)
+        rc = st->dtype == QS_C128 ? gate_reg<double, 2, true>(st, bits, m, false, cmask, cval)
+                                  : gate_reg<float, 2, true>(st, bits, m, false, cmask, cval);
+    else
+        rc = st->dtype == QS_C128 ? gate_reg<double, 4, true>(st, bits, m, false, cmask, cval)
+                                  : gate_reg<float, 4, true>(st, bits, m, false, cmask, cval);
     if (rc) return rc;
     QS_HIP(hipGetLastError(), "qpp::apply()");
     return QS_OK;

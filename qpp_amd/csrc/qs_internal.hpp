@@ -31,6 +31,7 @@ struct qs_state {
     bool qubits = true;          // all dims == 2
     uint32_t nbits = 0;          // log2(nelem) when qubits
     void* d = nullptr;           // device buffer
+    void* tab = nullptr;         // small tables of the call in progress (qs_gates.hip), on first use
     hipStream_t stream = nullptr;
     int device = 0;
     uint64_t elem_bytes() const { return dtype == QS_C128 ? 16 : 8; }
@@ -67,7 +68,7 @@ void set_thread_stream(hipStream_t s);
 // error-bounded parallel search
 bool force_exact_sampling();
 // measurement hook: QPP_AMD_GATEK_VALU=1 applies 4- and 5-qubit dense gates
-// on complex64 states with the VALU kernel instead of the MFMA one
+// on complex64 states with the kernel for any width (k_gatek)
 bool gatek_valu_forced();
 // qpp::measure_seq with the sampled basis index given (qs_measure.hip)
 int measure_seq_given(qs_state* st, uint32_t ntarget, const uint64_t* target,
@@ -98,6 +99,12 @@ int launch_gate1(qs_state* st, uint32_t bit, const double* m, uint64_t cmask,
 // k-bit dense gate, bits[0] the most significant digit of the gate index.
 int launch_gatek(qs_state* st, const uint32_t* bits, uint32_t k,
                  const double* m, uint64_t cmask, uint64_t cval, bool conj);
+
+// U rho U^dagger on k = 1 or 2 qubits of a density matrix in one pass: bits
+// are the column bits of the targets, then their row bits; the controls of
+// the rows (cmask[0], cval[0]) and of the columns.
+int launch_gate_rho(qs_state* st, const uint32_t* bits, uint32_t k, const double* m,
+                    const uint64_t (&cmask)[2], const uint64_t (&cval)[2]);
 
 // Mixed-radix (qudit) dense gate: element strides and digit ranges of the
 // gate's subsystems, spectator subsystems enumerated by the kernel.  Used
