@@ -250,7 +250,7 @@ int qs_sample(const qs_state* st, uint32_t ntarget, const uint64_t* target,
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc): same arguments, validation, results and
  * errors as qs_sample, but the call allocates nothing.  Its workspace is a
- * fixed array in device memory, one per GPU (about 16.4 MiB, held until the
+ * fixed array in device memory, one per GPU (about 8.4 MiB, held until the
  * process ends), so a call takes at most 2^20 basis states and 16384 shots
  * (larger ones fail with QS_ERR_OUT_OF_MEMORY before anything runs).  Every
  * shot is searched in the exact cumulative table.  Calls that overlap on one

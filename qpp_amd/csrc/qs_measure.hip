@@ -7,7 +7,7 @@
 //   cp_k = cp_{k-1} + q_k (sequential),    cp_{N-1} := 1,
 //   index = first k with cp_k >= u.
 // The GPU proceeds in two steps:
-//  1. k_chunk_sums / k_scan_chunks / k_search: a parallel prefix E_k of p in
+//  1. k_probs_sums / k_scan_chunks / k_search: a parallel prefix E_k of p in
 //     FP64 locates the candidate k with E_{k-1}/E < u <= E_k/E.  The
 //     candidate is accepted when u is farther than B from both edges, where
 //     B bounds |cp_k - E_k/E| over all k (bound_for()).
@@ -83,18 +83,43 @@ __device__ double block_sum(double v) {
     return r;
 }
 
-// per-chunk sums of p: one block per chunk
-__global__ __launch_bounds__(256) void k_chunk_sums(const double* __restrict__ p,
-                                                    uint64_t D,
-                                                    double* __restrict__ sums,
+// p and its per-chunk sums in one pass over the state, one block per chunk
+// (two passes over p: 103 us at 2^24 elements, this 66-91)
+template <typename T>
+__global__ __launch_bounds__(256) void k_probs_sums(const T* __restrict__ a, double* __restrict__ p,
+                                                    uint64_t D, int rho, double* __restrict__ sums,
                                                     uint64_t nchunks) {
     for (uint64_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-        const uint64_t b = c * kChunk;
+        const uint64_t b = c * kChunk + threadIdx.x;
+        T x[kChunk / 256];
+#pragma unroll
+        for (int j = 0; j < kChunk / 256; ++j) {
+            const uint64_t i = b + 256 * j;
+            x[j].x = 0;
+            x[j].y = 0;
+            if (i < D) x[j] = a[rho ? i + i * D : i];
+        }
         double v = 0;
-        for (uint64_t i = b + threadIdx.x; i < b + kChunk && i < D; i += 256) v += p[i];
+#pragma unroll
+        for (int j = 0; j < kChunk / 256; ++j) {
+            const uint64_t i = b + 256 * j;
+            const double q = rho ? static_cast<double>(x[j].x) : norm_exact(x[j].x, x[j].y);
+            if (i < D) p[i] = q;
+            v += q;
+        }
         v = block_sum(v);
         if (threadIdx.x == 0) sums[c] = v;
     }
+}
+
+// inclusive prefix sums over the lanes
+__device__ __forceinline__ double wave_incl_sum(double v, int lane) {
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) {
+        const double o = __shfl_up(v, m, 64);
+        if (lane >= m) v += o;
+    }
+    return v;
 }
 
 // exclusive prefix of the chunk sums, one block of 1024 threads; writes the
@@ -102,28 +127,28 @@ __global__ __launch_bounds__(256) void k_chunk_sums(const double* __restrict__ p
 __global__ __launch_bounds__(1024) void k_scan_chunks(const double* __restrict__ sums,
                                                       uint64_t nchunks,
                                                       double* __restrict__ prefix) {
-    __shared__ double part[1024];
+    __shared__ double part[16];
     const uint64_t per = (nchunks + 1023) / 1024;
     const uint64_t b = threadIdx.x * per;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     double v = 0;
     for (uint64_t i = b; i < b + per && i < nchunks; ++i) v += sums[i];
-    part[threadIdx.x] = v;
+    const double inc = wave_incl_sum(v, lane);
+    if (lane == 63) part[w] = inc;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double run = 0;
-        for (int t = 0; t < 1024; ++t) {
-            const double x = part[t];
-            part[t] = run;
-            run += x;
-        }
-        prefix[nchunks] = run;
+    double before = 0, total = 0;
+    for (int j = 0; j < 16; ++j) {
+        if (j == w) before = total;
+        total += part[j];
     }
-    __syncthreads();
-    double run = part[threadIdx.x];
+    double up = __shfl_up(inc, 1, 64);
+    if (lane == 0) up = 0;
+    double run = before + up;
     for (uint64_t i = b; i < b + per && i < nchunks; ++i) {
         prefix[i] = run;
         run += sums[i];
     }
+    if (threadIdx.x == 0) prefix[nchunks] = total;
 }
 
 // One wave per shot: binary search over chunk prefixes, then an in-chunk
@@ -151,30 +176,33 @@ __global__ __launch_bounds__(256) void k_search(const double* __restrict__ p,
         else
             hi = mid;
     }
-    // scan the chunk for the first element with E_k >= target
-    double run = prefix[lo];
+    // the 64 elements of the chunk that hold the first E_k >= target: each
+    // lane sums 64 consecutive ones; then those, one a lane
+    const uint64_t b = lo * kChunk;
+    double v = 0;
+#pragma unroll 16
+    for (int j = 0; j < kChunk / 64; ++j) {
+        const uint64_t i = b + uint64_t(lane) * (kChunk / 64) + j;
+        v += i < D ? p[i] : 0.0;
+    }
+    const double inc = wave_incl_sum(v, lane);
+    unsigned long long hit = __ballot(prefix[lo] + inc >= target);
     uint64_t found = D;  // D = not found in this chunk
     double e_prev = 0, e_at = 0;
-    const uint64_t b = lo * kChunk;
-    for (uint64_t s = b; s < b + kChunk && s < D; s += 64) {
+    if (hit) {
+        const int l0 = __ffsll(hit) - 1;
+        const double run = prefix[lo] + (l0 ? __shfl(inc, l0 - 1, 64) : 0.0);
+        const uint64_t s = b + uint64_t(l0) * (kChunk / 64);
         const uint64_t i = s + lane;
-        const double v = i < D ? p[i] : 0.0;
-        // inclusive wave scan
-        double inc = v;
-        for (int m = 1; m < 64; m <<= 1) {
-            const double o = __shfl_up(inc, m, 64);
-            if (lane >= m) inc += o;
-        }
-        const double e = run + inc;
-        const unsigned long long hit = __ballot(i < D && e >= target);
-        if (hit) {
+        const double x = i < D ? p[i] : 0.0;
+        const double e = run + wave_incl_sum(x, lane);
+        hit = __ballot(i < D && e >= target);
+        if (hit) {  // (rounding may leave the last one below the target)
             const int l = __ffsll(hit) - 1;
             found = s + l;
             e_at = __shfl(e, l, 64);
-            e_prev = __shfl(e - v, l, 64);
-            break;
+            e_prev = __shfl(e - x, l, 64);
         }
-        run += __shfl(inc, 63, 64);
     }
     if (lane == 0) {
         if (found == D) {
@@ -208,12 +236,14 @@ __global__ __launch_bounds__(256) void k_gather(const double* __restrict__ p,
 // t*kExV ...:
 //   k_ex_block_tr  one map per block, in the binade its approximate prefix
 //                  (k_scan_chunks) falls in;
-//   k_ex_chain     one wave walks the blocks in order carrying the exact sum:
-//                  64 blocks per step when their maps apply, otherwise the
-//                  block's own elements are scanned by the wave (wg_chunk);
-//   k_ex_expand    every block rebuilds its elements' sums from its exact
-//                  entry value (wg_chunk) and writes cp;
-//   k_ex_search    lower_bound(cp, u) per shot.
+//   k_ex_chain     one workgroup walks the blocks in order carrying the exact
+//                  sum over 1024 blocks a round while their maps apply; a
+//                  block whose map does not is scanned by its elements
+//                  (wg_chunk);
+//   k_ex_find      the block of every shot, by the blocks' exact entry values;
+//   k_ex_pick      rebuilds the cp of the blocks that have shots from their
+//                  entry values (wg_chunk), in LDS, and finds each shot's
+//                  lower_bound(cp, u) there.
 // The approximate prefix only picks the binade a block's map is built in;
 // a wrong pick sends the block to the element path and never changes a
 // result.  Element k of the summed sequence is p_k (S == nullptr) or
@@ -274,113 +304,161 @@ __global__ __launch_bounds__(256) void k_ex_block_tr(const double* __restrict__ 
     }
 }
 
-// One wave.  s_in[b] = exact sum before block b; s_in[nb] = the total.
-// The maps of the next 64 blocks are loaded while the current ones are
-// scanned.  A block whose map does not apply is summed by the wave itself
-// in two halves of 32 consecutive elements per lane, one scan each
-// (wg_chunk with one wave).
-__global__ __launch_bounds__(64) void k_ex_chain(const double* __restrict__ p, uint64_t D,
-                                                 const double* __restrict__ S, uint64_t nb,
-                                                 const qs_exact::Tr* __restrict__ T,
-                                                 const int* __restrict__ Eb,
-                                                 double* __restrict__ s_in) {
+// One workgroup.  s_in[b] = exact sum before block b; s_in[nb] = the total.
+// Each round carries the sum over up to 1024 blocks (four consecutive maps a
+// thread), as far as their maps apply; the block where they stop (its sum
+// leaves the binade, about a dozen per table) is then summed by its elements.
+// The first block, whose sum doubles at every power of two, is added in order
+// over its first kExHead elements, so that only a few doublings are left for
+// the scans.  A serial chain of scans, barriers and loads: with one wave, 64
+// blocks to a round, it took 416 us at 2^22 and 496 us at 2^24 elements,
+// 186 and 210 us so (a workgroup of 1024 was no faster than 350).
+constexpr int kExN = 256, kExMaps = 4, kExHead = 256;
+__global__ __launch_bounds__(kExN) void k_ex_chain(const double* __restrict__ p, uint64_t D,
+                                                   const double* __restrict__ S, uint64_t nb,
+                                                   const qs_exact::Tr* __restrict__ T,
+                                                   const int* __restrict__ Eb,
+                                                   double* __restrict__ s_in) {
     using namespace qs_exact;
-    __shared__ ChunkLds<64> L;
-    const int lane = threadIdx.x;
+    __shared__ ChunkLds<kExN> L;
+    __shared__ double head[kExHead];
+    const int t = threadIdx.x;
     const double sv = S ? *S : 1.0;
     double s = 0.0;
     uint64_t b = 0;
-    // maps of blocks pb + lane, loaded ahead
-    uint64_t pb = 0;
-    Tr tn = Tr{kTop, kTop};
-    int en = 0;
-    if (uint64_t(lane) < nb) {
-        tn = T[lane];
-        en = Eb[lane];
-    }
     while (b < nb) {
-        if (b != pb) {  // the group does not start where the prefetch assumed
-            pb = b;
-            if (pb + lane < nb) {
-                tn = T[pb + lane];
-                en = Eb[pb + lane];
-            }
-        }
-        const Tr tc = tn;
-        const int ec = en;
-        pb = b + 64;
-        if (pb + lane < nb) {
-            tn = T[pb + lane];
-            en = Eb[pb + lane];
-        }
         const int E = binade(s);
         const uint64_t m0 = mant(s);
-        const int cnt = nb - b < 64 ? int(nb - b) : 64;
-        const uint64_t j = b + lane;
-        const bool valid = lane < cnt && ec == E;
-        const Tr inc = wave_incl(valid ? tc : Tr{kTop, kTop}, lane);
-        const Tr ex = wave_excl(inc, lane);
-        const uint64_t mi = apply(m0, inc);
-        const unsigned long long bad = __ballot(lane < cnt && mi >= kTop);
-        const int f = bad ? __ffsll(bad) - 1 : cnt;  // blocks b .. b+f-1 apply
-        if (lane < f) s_in[j] = from_mant(apply(m0, ex), E);
-        if (f > 0) s = from_mant(apply(m0, shfl_tr(inc, f - 1)), E);
+        constexpr int B = kExN * kExMaps;
+        const int cnt = nb - b < B ? int(nb - b) : B;
+        Tr m[kExMaps], mine = identity();
+#pragma unroll
+        for (int k = 0; k < kExMaps; ++k) {
+            const int i = t * kExMaps + k;
+            m[k] = Tr{kTop, kTop};
+            if (b && i < cnt && Eb[b + i] == E) m[k] = T[b + i];
+        }
+#pragma unroll
+        for (int k = 0; k < kExMaps; ++k) mine = compose(mine, m[k]);
+        Tr ex, tot;
+        if (t == 0) {
+            L.first = cnt;
+            L.s = s;
+        }
+        wg_scan<kExN>(mine, L.tr, ex, tot);  // (its barriers order the writes above)
+        uint64_t mk = apply(m0, ex);
+#pragma unroll
+        for (int k = 0; k < kExMaps; ++k) {
+            const int i = t * kExMaps + k;
+            if (mk < kTop && i < cnt) {
+                const uint64_t before = mk;
+                mk = apply(mk, m[k]);
+                s_in[b + i] = from_mant(before, E);  // (the sum before the block, also where its map fails)
+                if (mk >= kTop)
+                    L.first = i;  // the only such block: the others start at kTop
+                if (i == cnt - 1 && mk < kTop) L.s = from_mant(mk, E);
+                if (mk >= kTop) L.s = from_mant(before, E);
+            }
+        }
+        __syncthreads();
+        const int f = L.first;  // blocks b .. b+f-1 apply
+        s = L.s;
+        __syncthreads();  // L is used again
         b += f;
         if (f < cnt) {
-            if (lane == 0) s_in[b] = s;
-            constexpr int V = kChunk / 128;  // two halves of 64 x 32 elements
-#pragma unroll 1
-            for (int h = 0; h < 2; ++h) {
-                const uint64_t i0 = b * kChunk + uint64_t(h) * (kChunk / 2) + uint64_t(lane) * V;
-                double x[V], out[V];
+            double x[kExV], out[kExV];
+            ex_load(p, D, S, sv, b, x);
+            if (b == 0) {
+                if (t < kExHead / kExV) {
 #pragma unroll
-                for (int k = 0; k < V; ++k) x[k] = i0 + k < D ? ex_elem(p, i0 + k, S, sv) : 0.0;
-                s = wg_chunk<64, V>(s, x, out, L);
+                    for (int k = 0; k < kExV; ++k) {
+                        head[t * kExV + k] = x[k];
+                        x[k] = 0.0;  // (adds nothing below)
+                    }
+                }
+                __syncthreads();
+#pragma unroll 16
+                for (int i = 0; i < kExHead; ++i) s = __dadd_rn(s, head[i]);
             }
+            s = wg_chunk<kExN, kExV>(s, x, out, L);
             b += 1;
         }
     }
-    if (lane == 0) s_in[nb] = s;
+    if (t == 0) s_in[nb] = s;
 }
 
-__global__ __launch_bounds__(256) void k_ex_expand(const double* __restrict__ p, uint64_t D,
-                                                   const double* __restrict__ S,
-                                                   const double* __restrict__ s_in,
-                                                   uint64_t nb, double* __restrict__ cp) {
-    using namespace qs_exact;
-    __shared__ ChunkLds<256> L;
-    const double sv = S ? *S : 1.0;
-    for (uint64_t b = blockIdx.x; b < nb; b += gridDim.x) {
-        double x[kExV], out[kExV];
-        ex_load(p, D, S, sv, b, x);
-        (void)wg_chunk<256, kExV>(s_in[b], x, out, L);
-        const uint64_t i0 = b * kChunk + uint64_t(threadIdx.x) * kExV;
-#pragma unroll
-        for (int j = 0; j < kExV; ++j) {
-            const uint64_t i = i0 + j;
-            if (i < D) cp[i] = i == D - 1 ? 1.0 : out[j];
-        }
-        __syncthreads();  // L is reused by the next block
-    }
-}
-
-// first k with cp[k] >= u[s] (cp[D-1] == 1 > u)
-__global__ __launch_bounds__(256) void k_ex_search(const double* __restrict__ cp, uint64_t D,
-                                                   const double* __restrict__ u,
-                                                   uint64_t nshots,
-                                                   uint64_t* __restrict__ idx) {
+// The block of every shot: the last one whose exact entry value is below u
+// (block 0 for u = 0); the first cp_k >= u lies in it.
+__global__ __launch_bounds__(256) void k_ex_find(const double* __restrict__ s_in, uint64_t nb,
+                                                 const double* __restrict__ u, uint64_t nshots,
+                                                 uint32_t* __restrict__ blk) {
     const uint64_t s = uint64_t(blockIdx.x) * 256 + threadIdx.x;
     if (s >= nshots) return;
     const double us = u[s];
-    uint64_t lo = 0, hi = D;
-    while (lo < hi) {
+    uint64_t lo = 0, hi = nb;  // s_in[lo] < us, or lo == 0
+    while (hi - lo > 1) {
         const uint64_t mid = lo + (hi - lo) / 2;
-        if (cp[mid] < us)
-            lo = mid + 1;
+        if (s_in[mid] < us)
+            lo = mid;
         else
             hi = mid;
     }
-    idx[s] = lo < D ? lo : D - 1;
+    blk[s] = static_cast<uint32_t>(lo);
+}
+
+// One block's exact table in LDS (the table of all blocks in HBM, and a
+// search of it, took 145 us at 2^24 elements, this 41-99), and in it the index of one shot (PERSHOT:
+// workgroup s takes shot s) or of all shots of the block (workgroup b).
+template <bool PERSHOT>
+__global__ __launch_bounds__(256) void k_ex_pick(const double* __restrict__ p, uint64_t D,
+                                                 const double* __restrict__ S,
+                                                 const double* __restrict__ s_in, uint64_t nb,
+                                                 const double* __restrict__ u, uint64_t nshots,
+                                                 const uint32_t* __restrict__ blk,
+                                                 uint64_t* __restrict__ idx) {
+    using namespace qs_exact;
+    __shared__ ChunkLds<256> L;
+    __shared__ double cp[kChunk + kChunk / kExV];  // one of padding per thread's run
+    __shared__ int any;
+    const double sv = *S;
+    for (uint64_t w = blockIdx.x; w < (PERSHOT ? nshots : nb); w += gridDim.x) {
+        const uint64_t b = PERSHOT ? blk[w] : w;
+        if (!PERSHOT) {
+            if (threadIdx.x == 0) any = 0;
+            __syncthreads();
+            for (uint64_t s = threadIdx.x; s < nshots; s += 256)
+                if (blk[s] == b) any = 1;
+            __syncthreads();
+            const int some = any;
+            __syncthreads();
+            if (!some) continue;
+        }
+        double x[kExV], out[kExV];
+        ex_load(p, D, S, sv, b, x);
+        (void)wg_chunk<256, kExV>(s_in[b], x, out, L);
+        const uint64_t i0 = b * kChunk;
+        const int n = D - i0 < uint64_t(kChunk) ? int(D - i0) : kChunk;
+#pragma unroll
+        for (int j = 0; j < kExV; ++j) {
+            const int e = int(threadIdx.x) * kExV + j;
+            cp[e + e / kExV] = i0 + e == D - 1 ? 1.0 : out[j];
+        }
+        __syncthreads();
+        for (uint64_t s = PERSHOT ? w + threadIdx.x * nshots : threadIdx.x; s < nshots; s += PERSHOT ? nshots : 256) {
+            if (!PERSHOT && blk[s] != b) continue;
+            const double us = u[s];
+            int lo = 0, hi = n;
+            while (lo < hi) {
+                const int mid = (lo + hi) / 2;
+                if (cp[mid + mid / kExV] < us)
+                    lo = mid + 1;
+                else
+                    hi = mid;
+            }
+            idx[s] = i0 + (lo < n ? lo : n - 1);
+        }
+        __syncthreads();  // L and cp are used again
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -486,6 +564,107 @@ __global__ __launch_bounds__(256) void k_contract(const T* __restrict__ in,
             x = ri + ci * Din;
         }
         out[y] = in[x];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// measured qubits, all at once
+// ---------------------------------------------------------------------------
+// qpp projects, renormalises and shrinks target by target.  With N_c the
+// weight (sum |a|^2, or the trace) of the elements that agree with the first
+// c results, target c's probability is N_c / N_(c-1) (N_0 = 1 as in qpp,
+// which does not renormalise before the first), and the state left is the
+// agreeing part over sqrt(N_k) (or N_k).  So one pass sums the weights of the
+// elements by how many leading results they agree with (bin c: 1 to k), and
+// one writes the state; elements that miss the first result are not read.
+// Measuring 4 of 24 qubits (complex128, without the sampling) took 620 us as
+// 12 passes with a wait for each target, 78 us so; 12 of 22, 540 -> 30 us.
+struct MeasBins {
+    uint32_t k;          // targets
+    uint32_t block[65];  // first workgroup of bin c + 1; [k]: all workgroups
+    uint64_t mask[64];   // index bits fixed in bin c + 1, and their values
+    uint64_t val[64];
+    uint64_t count[64];  // elements of bin c + 1
+};
+
+// x with zeros inserted at the set bits of mask
+__device__ __forceinline__ uint64_t deposit(uint64_t x, uint64_t mask) {
+    while (mask) {
+        const int b = __ffsll(static_cast<unsigned long long>(mask)) - 1;
+        const uint64_t low = (uint64_t{1} << b) - 1;
+        x = ((x & ~low) << 1) | (x & low);
+        mask &= mask - 1;
+    }
+    return x;
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void k_meas_sums(const T* __restrict__ a, uint64_t D, int rho, MeasBins mb,
+                                                   double* __restrict__ part) {
+    uint32_t c = 0;
+    while (blockIdx.x >= mb.block[c + 1]) ++c;
+    const uint64_t mask = mb.mask[c], val = mb.val[c], count = mb.count[c];
+    const uint64_t step = uint64_t(mb.block[c + 1] - mb.block[c]) * 256;
+    double v = 0;
+    for (uint64_t g = uint64_t(blockIdx.x - mb.block[c]) * 256 + threadIdx.x; g < count; g += 4 * step) {
+        T x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            x[j].x = 0;
+            x[j].y = 0;
+            if (g + j * step < count) {
+                const uint64_t i = deposit(g + j * step, mask) | val;
+                x[j] = a[rho ? i + i * D : i];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            v += rho ? double(x[j].x) : double(x[j].x) * x[j].x + double(x[j].y) * x[j].y;
+    }
+    v = block_sum(v);
+    if (threadIdx.x == 0) part[blockIdx.x] = v;
+}
+
+// N_1 .. N_k from the workgroups' sums: one wave per bin in turn, then the
+// suffix sums
+__global__ __launch_bounds__(256) void k_meas_final(const double* __restrict__ part, MeasBins mb,
+                                                    double* __restrict__ N) {
+    __shared__ double bin[64];
+    const int lane = threadIdx.x & 63;
+    for (uint32_t c = threadIdx.x / 64; c < mb.k; c += 4) {
+        double v = 0;
+        for (uint32_t b = mb.block[c] + lane; b < mb.block[c + 1]; b += 64) v += part[b];
+        v = wave_sum(v);
+        if (lane == 0) bin[c] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double n = 0;
+        for (uint32_t c = mb.k; c-- > 0;) N[c] = n += bin[c];
+    }
+}
+
+// the agreeing elements over c (ket: sqrt(N_k), rho: N_k); DESTROY: without
+// the measured bits, into out; else in place, the others zero (0 / c)
+template <typename T, bool DESTROY>
+__global__ __launch_bounds__(256) void k_meas_apply(const T* a, T* out, uint64_t n,
+                                                    uint64_t mask, uint64_t val, const double* __restrict__ Nk,
+                                                    int rho) {
+    using R = decltype(T{}.x);
+    const double c = rho ? *Nk : sqrt(*Nk);
+    const R zero = static_cast<R>(0.0 / c);
+    const uint64_t stride = uint64_t(gridDim.x) * 256;
+    for (uint64_t y = uint64_t(blockIdx.x) * 256 + threadIdx.x; y < n; y += stride) {
+        const uint64_t i = DESTROY ? deposit(y, mask) | val : y;
+        T r;
+        r.x = zero;
+        r.y = zero;
+        if (DESTROY || (i & mask) == val) {
+            const T v = a[i];
+            r.x = static_cast<R>(double(v.x) / c);
+            r.y = static_cast<R>(double(v.y) / c);
+        }
+        out[y] = r;
     }
 }
 
@@ -598,7 +777,6 @@ double bound_for(uint64_t N) {
 // (256-byte aligned segments).
 struct SampleWs {
     double* p;       // D probabilities
-    double* cp;      // D: the exact cumulative table
     double* sums;    // nchunks block sums
     double* prefix;  // nchunks + 1: their exclusive prefix and total
     qs_exact::Tr* T; // nchunks block maps
@@ -607,19 +785,19 @@ struct SampleWs {
     double* sq_in;   // nchunks + 1: the same for p / S
     double* u;       // nshots uniforms (then the gathered probabilities)
     uint64_t* idx;   // nshots indices
-    int* cert;       // nshots: decided by the approximate search
+    int* cert;       // nshots: decided by the approximate search, then the shot's block
 };
 
 constexpr size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
 // byte sizes of the SampleWs segments, in member order
-constexpr int kWsSegs = 11;
+constexpr int kWsSegs = 10;
 struct WsSizes {
     size_t seg[kWsSegs];
 };
 constexpr WsSizes ws_sizes(uint64_t D, uint64_t nshots) {
     const uint64_t nc = (D + kChunk - 1) / kChunk;
-    return WsSizes{{8 * D, 8 * D, 8 * nc, 8 * (nc + 1), sizeof(qs_exact::Tr) * nc, 4 * nc,
+    return WsSizes{{8 * D, 8 * nc, 8 * (nc + 1), sizeof(qs_exact::Tr) * nc, 4 * nc,
                     8 * (nc + 1), 8 * (nc + 1), 8 * nshots, 8 * nshots, 4 * nshots}};
 }
 constexpr size_t ws_bytes(uint64_t D, uint64_t nshots) {
@@ -639,22 +817,35 @@ size_t sample_ws_layout(uint64_t D, uint64_t nshots, unsigned char* base, Sample
     }
     if (w) {
         w->p = reinterpret_cast<double*>(at[0]);
-        w->cp = reinterpret_cast<double*>(at[1]);
-        w->sums = reinterpret_cast<double*>(at[2]);
-        w->prefix = reinterpret_cast<double*>(at[3]);
-        w->T = reinterpret_cast<qs_exact::Tr*>(at[4]);
-        w->Eb = reinterpret_cast<int*>(at[5]);
-        w->sp_in = reinterpret_cast<double*>(at[6]);
-        w->sq_in = reinterpret_cast<double*>(at[7]);
-        w->u = reinterpret_cast<double*>(at[8]);
-        w->idx = reinterpret_cast<uint64_t*>(at[9]);
-        w->cert = reinterpret_cast<int*>(at[10]);
+        w->sums = reinterpret_cast<double*>(at[1]);
+        w->prefix = reinterpret_cast<double*>(at[2]);
+        w->T = reinterpret_cast<qs_exact::Tr*>(at[3]);
+        w->Eb = reinterpret_cast<int*>(at[4]);
+        w->sp_in = reinterpret_cast<double*>(at[5]);
+        w->sq_in = reinterpret_cast<double*>(at[6]);
+        w->u = reinterpret_cast<double*>(at[7]);
+        w->idx = reinterpret_cast<uint64_t*>(at[8]);
+        w->cert = reinterpret_cast<int*>(at[9]);
     }
     return off;
 }
 
-// Builds the exact table in w.cp (k_ex_* above) and searches every shot in
-// it.  Needs w.p, w.prefix (k_chunk_sums + k_scan_chunks) and w.u.
+// w.p and w.sums
+int probs_sums(const qs_state* st, const SampleWs& w, uint64_t nchunks) {
+    const dim3 g(grid_for(nchunks, 1));
+    const int rho = st->kind == QS_RHO;
+    if (st->dtype == QS_C128)
+        hipLaunchKernelGGL(k_probs_sums<double2>, g, dim3(256), 0, st->stream,
+                           static_cast<const double2*>(st->d), w.p, st->D, rho, w.sums, nchunks);
+    else
+        hipLaunchKernelGGL(k_probs_sums<float2>, g, dim3(256), 0, st->stream,
+                           static_cast<const float2*>(st->d), w.p, st->D, rho, w.sums, nchunks);
+    QS_HIP(hipGetLastError(), "qpp::sample()");
+    return QS_OK;
+}
+
+// Every shot's index in the exact table (k_ex_* above).  Needs w.p, w.prefix
+// (k_probs_sums + k_scan_chunks) and w.u.
 int exact_table_search(const qs_state* st, const SampleWs& w, uint64_t nshots) {
     const uint64_t D = st->D;
     const uint64_t nb = (D + kChunk - 1) / kChunk;
@@ -662,15 +853,21 @@ int exact_table_search(const qs_state* st, const SampleWs& w, uint64_t nshots) {
     hipStream_t sm = st->stream;
     hipLaunchKernelGGL(k_ex_block_tr, dim3(g), dim3(256), 0, sm, w.p, D, nullptr, w.prefix, nb,
                        w.T, w.Eb);
-    hipLaunchKernelGGL(k_ex_chain, dim3(1), dim3(64), 0, sm, w.p, D, nullptr, nb, w.T, w.Eb,
+    hipLaunchKernelGGL(k_ex_chain, dim3(1), dim3(kExN), 0, sm, w.p, D, nullptr, nb, w.T, w.Eb,
                        w.sp_in);
     const double* S = w.sp_in + nb;
     hipLaunchKernelGGL(k_ex_block_tr, dim3(g), dim3(256), 0, sm, w.p, D, S, w.prefix, nb, w.T,
                        w.Eb);
-    hipLaunchKernelGGL(k_ex_chain, dim3(1), dim3(64), 0, sm, w.p, D, S, nb, w.T, w.Eb, w.sq_in);
-    hipLaunchKernelGGL(k_ex_expand, dim3(g), dim3(256), 0, sm, w.p, D, S, w.sq_in, nb, w.cp);
-    hipLaunchKernelGGL(k_ex_search, dim3(grid_for(nshots, 256)), dim3(256), 0, sm, w.cp, D, w.u,
-                       nshots, w.idx);
+    hipLaunchKernelGGL(k_ex_chain, dim3(1), dim3(kExN), 0, sm, w.p, D, S, nb, w.T, w.Eb, w.sq_in);
+    auto* blk = reinterpret_cast<uint32_t*>(w.cert);
+    hipLaunchKernelGGL(k_ex_find, dim3(grid_for(nshots, 256)), dim3(256), 0, sm, w.sq_in, nb, w.u, nshots, blk);
+    // a workgroup per shot or per block, whichever are fewer
+    if (nshots < nb)
+        hipLaunchKernelGGL(k_ex_pick<true>, dim3(grid_for(nshots, 1)), dim3(256), 0, sm, w.p, D, S, w.sq_in, nb,
+                           w.u, nshots, blk, w.idx);
+    else
+        hipLaunchKernelGGL(k_ex_pick<false>, dim3(g), dim3(256), 0, sm, w.p, D, S, w.sq_in, nb, w.u, nshots, blk,
+                           w.idx);
     QS_HIP(hipGetLastError(), "qpp::sample()");
     return QS_OK;
 }
@@ -691,7 +888,8 @@ int sample_device(const qs_state* st, const double* u_host, uint64_t nshots,
     const int rc = [&]() -> int {
         SampleWs w;
         sample_ws_layout(D, nshots, ws, &w);
-        if (int rc = probs_device(st, w.p)) return rc;
+        const uint64_t nchunks = (D + kChunk - 1) / kChunk;
+        if (int rc = probs_sums(st, w, nchunks)) return rc;
         if (D < 2) {  // a one-element table returns 0 (random.tcc:2700)
             for (uint64_t s = 0; s < nshots; ++s) out_idx[s] = 0;
             if (out_prob_host) {
@@ -702,11 +900,8 @@ int sample_device(const qs_state* st, const double* u_host, uint64_t nshots,
             }
             return QS_OK;
         }
-        const uint64_t nchunks = (D + kChunk - 1) / kChunk;
         QS_HIP(hipMemcpyAsync(w.u, u_host, nshots * 8, hipMemcpyHostToDevice, st->stream),
                "qpp::sample()");
-        hipLaunchKernelGGL(k_chunk_sums, dim3(grid_for(nchunks, 1)), dim3(256), 0, st->stream,
-                           w.p, D, w.sums, nchunks);
         hipLaunchKernelGGL(k_scan_chunks, dim3(1), dim3(1024), 0, st->stream, w.sums, nchunks,
                            w.prefix);
         const double B = bound_for(D);
@@ -756,7 +951,7 @@ int sample_device(const qs_state* st, const double* u_host, uint64_t nshots,
 // Allocation-free sampling (qs_sample_noalloc): the workspace of one call on
 // a state of at most kFixedMaxD basis states and kFixedMaxShots shots lives
 // in a file-scope device array.  Every GPU the library runs on holds its own
-// copy (about 16.4 MiB) until the process ends.  Its device address is
+// copy (about 8.4 MiB) until the process ends.  Its device address is
 // looked up once per device with hipGetSymbolAddress (the array's name is a
 // host-side stand-in, not a device address) and only that address is handed
 // to kernels and copies.  Nothing in it needs clearing: every segment is
@@ -802,7 +997,8 @@ int sample_exact_only(const qs_state* st, const double* u_host, uint64_t nshots,
     const uint64_t D = st->D;
     SampleWs w;
     sample_ws_layout(D, nshots, ws, &w);
-    if (int rc = probs_device(st, w.p)) return rc;
+    const uint64_t nchunks = (D + kChunk - 1) / kChunk;
+    if (int rc = probs_sums(st, w, nchunks)) return rc;
     if (D < 2) {  // a one-element table returns 0 (random.tcc:2700)
         if (idx_host)
             for (uint64_t s = 0; s < nshots; ++s) idx_host[s] = 0;
@@ -813,10 +1009,7 @@ int sample_exact_only(const qs_state* st, const double* u_host, uint64_t nshots,
         }
         return QS_OK;
     }
-    const uint64_t nchunks = (D + kChunk - 1) / kChunk;
     QS_HIP(hipMemcpyAsync(w.u, u_host, nshots * 8, hipMemcpyHostToDevice, st->stream), W);
-    hipLaunchKernelGGL(k_chunk_sums, dim3(grid_for(nchunks, 1)), dim3(256), 0, st->stream, w.p,
-                       D, w.sums, nchunks);
     hipLaunchKernelGGL(k_scan_chunks, dim3(1), dim3(1024), 0, st->stream, w.sums, nchunks,
                        w.prefix);
     if (int rc = exact_table_search(st, w, nshots)) return rc;
@@ -843,6 +1036,90 @@ int project(qs_state* st, uint64_t stride, uint64_t dim, uint64_t m) {
                            0, st->stream, static_cast<float2*>(st->d), st->nelem,
                            st->D, stride, dim, m, rho);
     QS_HIP(hipGetLastError(), "qpp::measure_seq()");
+    return QS_OK;
+}
+
+// dims after a destructive measurement (buffer already replaced)
+void set_dims(qs_state* st, std::vector<uint64_t> nd) {
+    if (nd.empty()) nd.push_back(1);
+    st->D = 1;
+    for (uint64_t d : nd) st->D *= d;
+    st->nelem = st->kind == QS_RHO ? st->D * st->D : st->D;
+    st->dims = nd;
+    st->qubits = std::all_of(nd.begin(), nd.end(), [](uint64_t d) { return d == 2; });
+    st->nbits = st->qubits ? static_cast<uint32_t>((st->kind == QS_RHO ? 2 : 1) * nd.size()) : 0;
+}
+
+// measure_seq_given on a qubit state: the results res of the targets, their
+// probabilities in the order qpp takes them (`order`)
+template <typename T>
+int measure_qubits(qs_state* st, const std::vector<uint64_t>& tv, const std::vector<uint64_t>& res,
+                   const std::vector<uint32_t>& order, bool destructive, std::vector<double>& ps) {
+    constexpr const char* W = "qpp::measure_seq()";
+    const uint32_t n = static_cast<uint32_t>(st->dims.size()), k = static_cast<uint32_t>(order.size());
+    const bool rho = st->kind == QS_RHO;
+    MeasBins mb{};
+    mb.k = k;
+    uint64_t mask = 0, val = 0;
+    for (uint32_t c = 0; c < k; ++c) {
+        const uint64_t bit = uint64_t{1} << (n - 1 - tv[order[c]]);
+        mask |= bit;
+        if (res[order[c]]) val |= bit;
+        mb.mask[c] = mask;
+        mb.val[c] = val;
+        mb.count[c] = uint64_t{1} << (n - c - 1);
+        if (c) {  // bin c agrees on the first c results and misses the next one
+            mb.mask[c - 1] = mask;
+            mb.val[c - 1] = val ^ bit;
+            mb.count[c - 1] = uint64_t{1} << (n - c - 1);
+        }
+    }
+    for (uint32_t c = 0; c < k; ++c)
+        mb.block[c + 1] = mb.block[c] + static_cast<uint32_t>(std::min<uint64_t>(1024, (mb.count[c] + 4095) / 4096));
+    double* part = nullptr;
+    const uint32_t nblocks = mb.block[k];
+    QS_HIP(hipMallocAsync(reinterpret_cast<void**>(&part), sizeof(double) * (nblocks + k), st->stream), W);
+    double* N = part + nblocks;
+    auto* a = static_cast<T*>(st->d);
+    hipLaunchKernelGGL(k_meas_sums<T>, dim3(nblocks), dim3(256), 0, st->stream, a, st->D, int(rho), mb, part);
+    hipLaunchKernelGGL(k_meas_final, dim3(1), dim3(256), 0, st->stream, part, mb, N);
+    uint64_t emask = mask, eval = val;  // of the element index
+    if (rho) {
+        emask |= mask << n;
+        eval |= val << n;
+    }
+    void* nbuf = nullptr;
+    hipError_t e = hipSuccess;
+    if (destructive) {
+        const uint64_t nout = st->nelem >> (rho ? 2 * k : k);
+        e = hipMallocAsync(&nbuf, nout * st->elem_bytes(), st->stream);
+        if (e == hipSuccess)
+            hipLaunchKernelGGL((k_meas_apply<T, true>), dim3(grid_for(nout, 256)), dim3(256), 0, st->stream, a,
+                               static_cast<T*>(nbuf), nout, emask, eval, N + k - 1, int(rho));
+    } else {
+        hipLaunchKernelGGL((k_meas_apply<T, false>), dim3(grid_for(st->nelem, 256)), dim3(256), 0, st->stream, a, a,
+                           st->nelem, emask, eval, N + k - 1, int(rho));
+    }
+    std::vector<double> h(k);
+    if (e == hipSuccess) e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(h.data(), N, sizeof(double) * k, hipMemcpyDeviceToHost, st->stream);
+    (void)hipFreeAsync(part, st->stream);
+    const hipError_t e2 = hipStreamSynchronize(st->stream);
+    if (e == hipSuccess) e = e2;
+    if (e != hipSuccess) {
+        if (nbuf) (void)hipFreeAsync(nbuf, st->stream);
+        return qs::fail_hip(e, W);
+    }
+    if (destructive) {
+        (void)hipFreeAsync(st->d, st->stream);
+        st->d = nbuf;
+        std::vector<uint64_t> nd;
+        for (uint32_t q = 0; q < n; ++q)
+            if (!((mask >> (n - 1 - q)) & 1)) nd.push_back(2);
+        set_dims(st, nd);
+        if (nd.empty()) st->qubits = false, st->nbits = 0;
+    }
+    for (uint32_t c = 0; c < k; ++c) ps[order[c]] = c ? h[c] / h[c - 1] : h[c];
     return QS_OK;
 }
 
@@ -1068,7 +1345,16 @@ int qs::measure_seq_given(qs_state* st, uint32_t ntarget, const uint64_t* target
     const bool rho = st->kind == QS_RHO;
     std::vector<uint32_t> order(ntarget);
     std::iota(order.begin(), order.end(), 0u);
-    if (rho && n0 <= 10) {
+    // the order qpp projects in: as given for small density matrices
+    // (instruments.hpp:1039-1054), else from the last subsystem when
+    // destructive
+    if (destructive && !(rho && n0 <= 10))
+        std::sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return tv[a] > tv[b]; });
+    if (st->qubits && ntarget > 0) {
+        if (int rc = st->dtype == QS_C128 ? measure_qubits<double2>(st, tv, res, order, destructive != 0, ps)
+                                          : measure_qubits<float2>(st, tv, res, order, destructive != 0, ps))
+            return rc;
+    } else if (rho && n0 <= 10) {
         // instruments.hpp:1039-1054: project in the given order, then one
         // ptrace over all targets
         for (uint32_t cnt = 0; cnt < ntarget; ++cnt) {
@@ -1088,9 +1374,6 @@ int qs::measure_seq_given(qs_state* st, uint32_t ntarget, const uint64_t* target
                 if (int rc = contract(st, tv[k], res[k])) return rc;
         }
     } else {
-        if (destructive)
-            std::sort(order.begin(), order.end(),
-                      [&](uint32_t a, uint32_t b) { return tv[a] > tv[b]; });
         for (uint32_t cnt = 0; cnt < ntarget; ++cnt) {
             const uint32_t ip = order[cnt];
             const uint64_t i = tv[ip];
