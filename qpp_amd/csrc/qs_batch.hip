@@ -286,34 +286,70 @@ __global__ __launch_bounds__(kThreads) void k_traj(cxt<R>* __restrict__ ws, uint
         const uint64_t N = uint64_t{1} << c.nb;
         const uint64_t blk = N / kThreads;  // nb >= 11 -> blk >= 8
         const uint64_t xm = ti.xmask;
-        {
-            double s = 0;
-            const uint64_t i0 = uint64_t(t) * blk;
-            for (uint64_t i = i0; i < i0 + blk; ++i) s += pnorm(a[i ^ xm]);
-            pre[t + 1] = s;
+        const double u = u_traj;
+        const uint32_t lane = t & 63;
+        // sums of the 256 runs of blk outcomes: a wave takes four runs at a
+        // time, its lanes consecutive outcomes
+        for (uint32_t r0 = (t >> 6) * 64; r0 < (t >> 6) * 64 + 64; r0 += 4) {
+            double s[4] = {0, 0, 0, 0};
+            for (uint64_t i = lane; i < blk; i += 64)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) s[j] += pnorm(a[((r0 + j) * blk + i) ^ xm]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                for (int m = 32; m > 0; m >>= 1) s[j] += __shfl_xor(s[j], m, 64);
+                if (lane == 0) pre[r0 + j + 1] = s[j];
+            }
         }
         __syncthreads();
-        if (t == 0) {
-            pre[0] = 0;
-            for (int j = 1; j <= kThreads; ++j) pre[j] = pre[j - 1] + pre[j];
-            const double total = pre[kThreads];
-            const double u = u_traj;
-            const double target = u * total;
-            int b = 0;
-            while (b < kThreads - 1 && pre[b + 1] < target) ++b;
-            double cc = pre[b], cprev = cc;
+        // prefix over the threads' values v: pre[0..256]; and the first
+        // thread whose prefix reaches the target (the last one if none does)
+        auto prefix_and_find = [&](double v, double start, double target_of_total, bool relative) {
+            double inc = v;
+            for (int m = 1; m < 64; m <<= 1) {
+                const double o = __shfl_up(inc, m, 64);
+                if (lane >= uint32_t(m)) inc += o;
+            }
+            __shared__ double wsum[kThreads / 64];
+            if (t == 0) s_k = kThreads - 1;
+            if (lane == 63) wsum[t >> 6] = inc;
+            __syncthreads();
+            double before = start, all = start;
+            for (uint32_t w = 0; w < kThreads / 64; ++w) {
+                if (w == (t >> 6)) before = all;
+                all += wsum[w];
+            }
+            pre[t + 1] = before + inc;
+            if (t == 0) pre[0] = start;
+            const double target = relative ? target_of_total * all : target_of_total;
+            if (before + inc >= target) atomicMin(&s_k, t);
+            __syncthreads();
+        };
+        prefix_and_find(pre[t + 1], 0.0, u, true);
+        const double total = pre[kThreads];
+        const double target = u * total;
+        const uint64_t i1 = s_k * blk;  // the run that holds it
+        const double e1 = pre[s_k];
+        __syncthreads();
+        // within the run: a thread each for per consecutive outcomes
+        const uint64_t per = (blk + kThreads - 1) / kThreads;
+        double v = 0;
+        for (uint64_t i = t * per; i < (t + 1) * per && i < blk; ++i) v += pnorm(a[(i1 + i) ^ xm]);
+        prefix_and_find(v, e1, target, false);
+        if (t == s_k) {
+            double cc = pre[t], cprev = cc;
             uint64_t idx = N;
-            for (uint64_t i = uint64_t(b) * blk; i < uint64_t(b + 1) * blk; ++i) {
+            for (uint64_t i = t * per; i < (t + 1) * per && i < blk; ++i) {
                 cprev = cc;
-                cc += pnorm(a[i ^ xm]);
+                cc += pnorm(a[(i1 + i) ^ xm]);
                 if (cc >= target) {
-                    idx = i;
+                    idx = i1 + i;
                     break;
                 }
             }
             // distance of the exact libstdc++ table from ours, relative to
             // the total: sequential sum and partial sums of N terms on its
-            // side, block sums + prefix + block scan on ours
+            // side, run sums and their prefixes (fewer terms) on ours
             const double bound =
                 2.0 * (2.0 * double(N) + 2.0 * double(blk) + 2.0 * kThreads + 8.0) * kUr * total;
             const bool certain = !force_exact && idx < N &&
@@ -338,7 +374,7 @@ __global__ __launch_bounds__(kThreads) void k_traj(cxt<R>* __restrict__ ws, uint
             const uint64_t idx = s_idx;
             TrajOut o;
             o.index = idx;
-            o.prob = pnorm(a[idx ^ xm]) / pre[kThreads];
+            o.prob = pnorm(a[idx ^ xm]) / total;
             o.exact = s_certain ? 0 : 1;
             o.pad = 0;
             out[tr] = o;
@@ -869,15 +905,48 @@ int qs_batch_plan(const qs_batch* b, uint32_t circuit, uint64_t seed, double noi
 
 namespace {
 
-// Trajectories of at least this many qubits run pass by pass over all their
-// tiles (k_traj_pass, one workgroup per tile of each such state) before
+// Trajectories of at least kWideBits qubits always run pass by pass over all
+// their tiles (k_traj_pass, one workgroup per tile of each such state) before
 // k_traj measures them: one workgroup streaming a state of 2^20 amplitudes
-// and more tile after tile is bound by its own latency.  The environment
-// variable QPP_AMD_TRAJ_WIDE_BITS sets another threshold (64: none).
-uint32_t wide_bits() {
+// and more tile after tile is bound by its own latency.  Smaller ones do
+// where that is expected to take no longer than a workgroup each
+// (small_go_wide).  The environment variable QPP_AMD_TRAJ_WIDE_BITS sets
+// another threshold and turns the rule off (64: none).
+constexpr uint32_t kWideBits = 18;
+
+bool wide_bits_set(uint32_t* bits) {
     const char* v = std::getenv("QPP_AMD_TRAJ_WIDE_BITS");
-    if (!v || !*v) return 18;
-    return static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
+    if (!v || !*v) return false;
+    *bits = static_cast<uint32_t>(std::strtoul(v, nullptr, 10));
+    return true;
+}
+
+// Both ways in units of one workgroup's tile and pass (about 40 us of a
+// complex128 tile, launch included): pass by pass, the launches of every
+// circuit follow each other, each as many rounds of the chip's resident
+// workgroups (three per CU) as its tiles take; with a workgroup each, the
+// longest trajectory or two rounds' worth per CU.  192 trajectories of 16
+// qubits: 16.3 -> 5.7 ms (complex64 10.9 -> 3.2), 16 of them 16.1 -> 1.2 ms,
+// 3000 of 12 qubits 6.5 -> 4.7 ms; many circuits with one trajectory each
+// keep their workgroups.
+bool small_go_wide(const qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, uint64_t ncu) {
+    std::vector<uint64_t> count(b->cls.size(), 0);
+    for (uint64_t i = 0; i < ntraj; ++i) ++count[circuit_of[i]];
+    double wide = 0, longest = 0, all = 0;
+    for (size_t c = 0; c < count.size(); ++c) {
+        const Cls& k = b->cls[c];
+        if (!count[c] || k.nb >= kWideBits) continue;
+        double launches = 0, tiles = 0;
+        for (const FPass& p : k.P.passes) {
+            if (p.phase_begin >= p.phase_end || p.ntiles == 0) return false;
+            launches += double((count[c] * p.ntiles + 3 * ncu - 1) / (3 * ncu));
+            tiles += double(p.ntiles);
+        }
+        wide += launches;
+        longest = std::max(longest, tiles);
+        all += tiles * double(count[c]);
+    }
+    return wide <= std::max(longest, all / double(2 * ncu));
 }
 
 // One launch of k_traj over ntraj trajectories (arguments validated by the
@@ -927,7 +996,12 @@ int run_impl(qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, const uint
     std::vector<uint32_t> order(ntraj);
     std::iota(order.begin(), order.end(), 0u);
     // wide trajectories, grouped by circuit: their passes run before k_traj
-    const uint32_t wbits = wide_bits();
+    int dev = 0, ncu = 0;
+    QS_HIP(hipGetDevice(&dev), W);
+    QS_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), W);
+    uint32_t wbits = 0;
+    if (!wide_bits_set(&wbits))
+        wbits = small_go_wide(b, ntraj, circuit_of, std::max(1, ncu)) ? 0 : kWideBits;
     std::vector<uint32_t> wide;
     std::vector<char> is_wide(ntraj, 0);
     for (uint64_t i = 0; i < ntraj; ++i) {
@@ -964,9 +1038,6 @@ int run_impl(qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, const uint
                 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<float, 8>, kThreads, shmem)
                 : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<float, 16>, kThreads, shmem);
     if (e != hipSuccess) return qs::fail_hip(e, W);
-    int dev = 0, ncu = 0;
-    QS_HIP(hipGetDevice(&dev), W);
-    QS_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), W);
     const uint64_t grid = std::max<uint64_t>(1, std::min<uint64_t>(ntraj, uint64_t(std::max(1, per_cu)) * ncu));
     const uint64_t slot = uint64_t{1} << maxnb;
     const size_t ws_bytes = dst ? 0 : size_t(grid) * slot * es;
@@ -1155,7 +1226,31 @@ int qs_batch_run(qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, const 
     if (!(noise_p <= 1.0)) return fail(QS_ERR_OUT_OF_RANGE, W, "noise_p");
     for (uint64_t i = 0; i < ntraj; ++i)
         if (circuit_of[i] >= b->cls.size()) return fail(QS_ERR_OUT_OF_RANGE, W, "circuit_of");
-    return run_impl(b, ntraj, circuit_of, seeds, noise_p, nullptr, out_index, out_prob);
+    // Pass by pass, every trajectory has a state of its own: those of fewer
+    // than kWideBits qubits are taken in runs of at most 4 GiB of states
+    // (some thousand trajectories at least).
+    constexpr uint64_t kMost = uint64_t{4} << 30;
+    uint64_t exact = 0;
+    double host = 0, device = 0;
+    for (uint64_t i0 = 0, i1; i0 < ntraj; i0 = i1) {
+        uint64_t bytes = 0;
+        for (i1 = i0; i1 < ntraj; ++i1) {
+            const uint32_t nb = b->cls[circuit_of[i1]].nb;
+            const uint64_t need = nb < kWideBits ? (b->dtype == QS_C128 ? 16u : 8u) * (uint64_t{1} << nb) : 0;
+            if (bytes + need > kMost) break;
+            bytes += need;
+        }
+        if (int rc = run_impl(b, i1 - i0, circuit_of + i0, seeds + i0, noise_p, nullptr,
+                              out_index ? out_index + i0 : nullptr, out_prob ? out_prob + i0 : nullptr))
+            return rc;
+        exact += b->last_exact;
+        host += b->last_host_ms;
+        device += b->last_device_ms;
+    }
+    b->last_exact = exact;
+    b->last_host_ms = host;
+    b->last_device_ms = device;
+    return QS_OK;
 }
 
 // The gate steps of circuit circuit_of[i] applied to |0..0> into out[i] (a

@@ -198,6 +198,21 @@ def test_wide_trajectories_more_than_one_launch_row(monkeypatch):
 
 
 @gpu
+@pytest.mark.parametrize("n,ntr,depth", [(12, 1, 3), (13, 300, 2), (16, 40, 2), (17, 2100, 1)])
+def test_small_trajectories_by_rule(monkeypatch, n, ntr, depth):
+    """Which way trajectories below the wide threshold run is chosen by
+    their number and tiles, and more than 4 GiB of their states are taken in
+    several runs; outcomes equal the persistent launch's bit for bit."""
+    b = qa.Batch([noisy_circuit(n, depth, seed=91), noisy_circuit(12, 2, seed=92)], dtype=qa.C128)
+    cof = np.array([int(i % 7 == 3) for i in range(ntr)], dtype=np.uint32)
+    seeds = np.arange(ntr, dtype=np.uint64) + 99
+    i0, p0 = b.run(cof, seeds, 0.01)
+    monkeypatch.setenv("QPP_AMD_TRAJ_WIDE_BITS", "64")
+    i1, p1 = b.run(cof, seeds, 0.01)
+    assert np.array_equal(i0, i1) and np.array_equal(p0, p1)
+
+
+@gpu
 def test_wide_trajectories_vs_oracle_engine(orc, monkeypatch):
     monkeypatch.setenv("QPP_AMD_TRAJ_WIDE_BITS", "12")
     circs = [noisy_circuit(12, 3, seed=81, cz=True), noisy_circuit(13, 2, seed=82, extra=True)]
