@@ -315,6 +315,43 @@ int gate_dispatch(qs_state* st, const double* A, uint64_t dimA,
 
 }  // namespace
 
+int qs::create_uninit(qs_dtype dtype, qs_kind kind, uint32_t ndims, const uint64_t* dims, qs_state** out) {
+    if (!out) return fail(QS_ERR_INVALID_HANDLE, "qs_state_create", "out");
+    *out = nullptr;
+    if (dtype != QS_C128 && dtype != QS_C64)
+        return fail(QS_ERR_TYPE_MISMATCH, "qs_state_create", "dtype");
+    if (kind != QS_KET && kind != QS_RHO)
+        return fail(QS_ERR_MATRIX_NOT_SQUARE_NOR_CVECTOR, "qs_state_create", "kind");
+    const auto dv = to_vec(dims, ndims);
+    // check_dims, internal/util.hpp:158-166
+    if (dv.empty() || std::find(dv.begin(), dv.end(), uint64_t{0}) != dv.end())
+        return fail(QS_ERR_DIMS_INVALID, "qs_state_create", "dims");
+    if (int rc = qs::ensure_device()) return rc;
+    auto* st = new qs_state;
+    st->dtype = dtype;
+    st->kind = kind;
+    st->dims = dv;
+    st->D = 1;
+    for (uint64_t d : dv) {
+        if (st->D > (uint64_t{1} << 40) / d) {
+            delete st;
+            return fail(QS_ERR_OUT_OF_RANGE, "qs_state_create", "dims");
+        }
+        st->D *= d;
+    }
+    st->nelem = kind == QS_KET ? st->D : st->D * st->D;
+    st->qubits = std::all_of(dv.begin(), dv.end(), [](uint64_t d) { return d == 2; });
+    st->nbits = st->qubits ? static_cast<uint32_t>((kind == QS_KET ? 1 : 2) * dv.size()) : 0;
+    st->stream = qs::current_stream();
+    hipError_t e = hipMallocAsync(&st->d, st->bytes(), st->stream);
+    if (e != hipSuccess) {
+        delete st;
+        return qs::fail_hip(e, "qs_state_create");
+    }
+    *out = st;
+    return QS_OK;
+}
+
 extern "C" {
 
 const char* qs_last_error(void) { return qs::g_last_error.c_str(); }
@@ -367,44 +404,12 @@ int qs_profile_end(double* ms) {
 
 int qs_state_create(qs_dtype dtype, qs_kind kind, uint32_t ndims,
                     const uint64_t* dims, qs_state** out) {
-    if (!out) return fail(QS_ERR_INVALID_HANDLE, "qs_state_create", "out");
-    *out = nullptr;
-    if (dtype != QS_C128 && dtype != QS_C64)
-        return fail(QS_ERR_TYPE_MISMATCH, "qs_state_create", "dtype");
-    if (kind != QS_KET && kind != QS_RHO)
-        return fail(QS_ERR_MATRIX_NOT_SQUARE_NOR_CVECTOR, "qs_state_create", "kind");
-    const auto dv = to_vec(dims, ndims);
-    // check_dims, internal/util.hpp:158-166
-    if (dv.empty() || std::find(dv.begin(), dv.end(), uint64_t{0}) != dv.end())
-        return fail(QS_ERR_DIMS_INVALID, "qs_state_create", "dims");
-    if (int rc = qs::ensure_device()) return rc;
-    auto* st = new qs_state;
-    st->dtype = dtype;
-    st->kind = kind;
-    st->dims = dv;
-    st->D = 1;
-    for (uint64_t d : dv) {
-        if (st->D > (uint64_t{1} << 40) / d) {
-            delete st;
-            return fail(QS_ERR_OUT_OF_RANGE, "qs_state_create", "dims");
-        }
-        st->D *= d;
-    }
-    st->nelem = kind == QS_KET ? st->D : st->D * st->D;
-    st->qubits = std::all_of(dv.begin(), dv.end(), [](uint64_t d) { return d == 2; });
-    st->nbits = st->qubits ? static_cast<uint32_t>((kind == QS_KET ? 1 : 2) * dv.size()) : 0;
-    st->stream = qs::current_stream();
-    hipError_t e = hipMallocAsync(&st->d, st->bytes(), st->stream);
-    if (e != hipSuccess) {
-        delete st;
-        return qs::fail_hip(e, "qs_state_create");
-    }
-    if (int rc = set_basis(st, 0)) {
-        (void)hipFreeAsync(st->d, st->stream);
-        delete st;
+    if (int rc = qs::create_uninit(dtype, kind, ndims, dims, out)) return rc;
+    if (int rc = set_basis(*out, 0)) {
+        qs_state_destroy(*out);
+        *out = nullptr;
         return rc;
     }
-    *out = st;
     return QS_OK;
 }
 
@@ -421,9 +426,8 @@ int qs_state_destroy(qs_state* st) {
 int qs_state_clone(const qs_state* st, qs_state** out) {
     if (!valid(st) || !out) return fail(QS_ERR_INVALID_HANDLE, "qs_state_clone");
     const qs::StreamScope on(st->stream);  // the copy lives on the source's stream
-    if (int rc = qs_state_create(st->dtype, st->kind,
-                                 static_cast<uint32_t>(st->dims.size()),
-                                 st->dims.data(), out))
+    if (int rc = qs::create_uninit(st->dtype, st->kind, static_cast<uint32_t>(st->dims.size()),
+                                   st->dims.data(), out))
         return rc;
     QS_HIP(hipMemcpyAsync((*out)->d, st->d, st->bytes(), hipMemcpyDeviceToDevice,
                           st->stream),

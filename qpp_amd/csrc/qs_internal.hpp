@@ -85,6 +85,9 @@ struct StreamScope {
     ~StreamScope();
 };
 
+// qs_state_create without the fill, for a state that is written whole next
+int create_uninit(qs_dtype dtype, qs_kind kind, uint32_t ndims, const uint64_t* dims, qs_state** out);
+
 // ---------------------------------------------------------------------------
 // kernel launchers (defined in the .hip files).  `m` is a column-major
 // complex128 matrix (interleaved re/im).  Bit positions are LSB numbering of

@@ -19,10 +19,12 @@
 #include <numeric>
 #include <vector>
 
+#include "qs_digits.hpp"
 #include "qs_internal.hpp"
 
 namespace {
 
+using namespace qs_digits;
 using qs::fail;
 
 // ---------------------------------------------------------------------------
@@ -130,65 +132,55 @@ __global__ __launch_bounds__(256) void k_bitperm(const T* __restrict__ in,
 }
 
 // ---------------------------------------------------------------------------
-// mixed-radix digit permutation: output digit k (dims odim[k], stride ostr)
-// takes the input digit at input stride istr[k]
+// mixed-radix digit permutation: output digit k takes the input digit at
+// input stride g.str[k], the digits by 32-bit reciprocals.  The gather of
+// single elements bounds it: 14 qutrits complex128 take 67-72 us at any cost
+// of the digits (2.1 TB/s).
 // ---------------------------------------------------------------------------
-struct DigitPerm {
-    uint32_t nd;
-    uint64_t odim[80];
-    uint64_t istr[80];
-};
-
-template <typename T>
-__global__ __launch_bounds__(256) void k_digitperm(const T* __restrict__ in,
-                                                   T* __restrict__ out,
-                                                   uint64_t n, DigitPerm dp) {
-    const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
-    for (uint64_t y = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; y < n;
-         y += stride) {
-        uint64_t rem = y, x = 0;
-        for (int k = int(dp.nd) - 1; k >= 0; --k) {
-            x += (rem % dp.odim[k]) * dp.istr[k];
-            rem /= dp.odim[k];
+template <typename T, typename DG>
+__global__ __launch_bounds__(256) void k_digitperm(const T* __restrict__ in, T* __restrict__ out,
+                                                   uint64_t n, DG g) {
+    const uint64_t stride = uint64_t(gridDim.x) * 256;
+    for (uint64_t y = uint64_t(blockIdx.x) * 256 + threadIdx.x; y < n; y += 4 * stride) {
+        T v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            // past the end: the last element, not stored
+            const uint64_t at = y + j * stride < n ? y + j * stride : n - 1;
+            v[j] = in[offset_of(g, typename DG::Index(at))];
         }
-        out[y] = in[x];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (y + j * stride < n) out[y + j * stride] = v[j];
     }
 }
 
 // ---------------------------------------------------------------------------
 // ket partial transpose: out(i, j) = psi(r) conj(psi(c)) with r, c the row
-// and column indices after swapping the target digits (mixed radix)
+// and column indices after swapping the target digits: with S(i) the target
+// digits' part of an index, r = i - S(i) + S(j) and c = j - S(j) + S(i).  A
+// thread takes one row and 16 columns, so S costs little and the writes bound
+// it (12 qubits complex128: 385 us with the digits of every element by 64-bit
+// division, TODO us).
 // ---------------------------------------------------------------------------
-struct KetPT {
-    uint32_t n;
-    uint64_t dim[40];
-    uint64_t stride[40];
-    uint8_t swap[40];
-    uint64_t D;
-};
+constexpr uint32_t kPtCols = 16;
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_ket_pt(const T* __restrict__ psi,
-                                                T* __restrict__ out, KetPT p) {
-    const uint64_t total = p.D * p.D;
-    const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
-    for (uint64_t y = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; y < total;
-         y += stride) {
-        const uint64_t i = y % p.D, j = y / p.D;
-        uint64_t ri = i, rj = j, r = 0, c = 0;
-        for (int k = int(p.n) - 1; k >= 0; --k) {
-            const uint64_t di = ri % p.dim[k], dj = rj % p.dim[k];
-            ri /= p.dim[k];
-            rj /= p.dim[k];
-            r += (p.swap[k] ? dj : di) * p.stride[k];
-            c += (p.swap[k] ? di : dj) * p.stride[k];
+template <typename T, typename DG>
+__global__ __launch_bounds__(256) void k_ket_pt(const T* __restrict__ psi, T* __restrict__ out, uint64_t D,
+                                                DG swapped) {
+    using Ix = typename DG::Index;
+    const uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= D) return;
+    const uint64_t si = offset_of(swapped, Ix(i));
+    for (uint64_t j0 = uint64_t(blockIdx.y) * kPtCols; j0 < D; j0 += uint64_t(gridDim.y) * kPtCols)
+        for (uint64_t j = j0; j < j0 + kPtCols && j < D; ++j) {
+            const uint64_t sj = offset_of(swapped, Ix(j));
+            const T a = psi[i - si + sj], b = psi[j - sj + si];
+            T v;
+            v.x = a.x * b.x + a.y * b.y;
+            v.y = a.y * b.x - a.x * b.y;
+            out[i + j * D] = v;
         }
-        const T a = psi[r], b = psi[c];
-        T v;
-        v.x = a.x * b.x + a.y * b.y;
-        v.y = a.y * b.x - a.x * b.y;
-        out[y] = v;
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -224,8 +216,7 @@ int make_out(const qs_state* st, qs_kind kind, const std::vector<uint64_t>& dims
              qs_state** out) {
     // created on `st`'s stream: kernels reading `st` write it in stream order
     const qs::StreamScope on(st->stream);
-    return qs_state_create(st->dtype, kind, static_cast<uint32_t>(dims.size()), dims.data(),
-                           out);
+    return qs::create_uninit(st->dtype, kind, static_cast<uint32_t>(dims.size()), dims.data(), out);
 }
 
 // out[y] = in[G(y)], src[b] = input bit of output bit b
@@ -340,24 +331,42 @@ int bitperm(const qs_state* in, qs_state* out, const std::vector<uint32_t>& src)
 }
 
 template <typename T>
-int launch_digitperm(const qs_state* in, qs_state* out, const DigitPerm& dp) {
-    hipLaunchKernelGGL(k_digitperm<T>, dim3(grid_for(out->nelem, 256)), dim3(256), 0,
-                       in->stream, static_cast<const T*>(in->d),
-                       static_cast<T*>(out->d), out->nelem, dp);
+int launch_digitperm(const qs_state* in, qs_state* out, const DigitList& list) {
+    const dim3 g(grid_for(out->nelem, 1024));
+    const T* src = static_cast<const T*>(in->d);
+    T* dst = static_cast<T*>(out->d);
+    Digits fit;
+    if (digits_fit(list, &fit))
+        hipLaunchKernelGGL((k_digitperm<T, Digits>), g, dim3(256), 0, in->stream, src, dst, out->nelem, fit);
+    else
+        hipLaunchKernelGGL((k_digitperm<T, WideDigits>), g, dim3(256), 0, in->stream, src, dst, out->nelem,
+                           wide_digits(list));
     QS_HIP(hipGetLastError(), "qpp_amd::digitperm");
     return QS_OK;
 }
 
-int digitperm(const qs_state* in, qs_state* out, const DigitPerm& dp) {
-    return in->dtype == QS_C128 ? launch_digitperm<double2>(in, out, dp)
-                                : launch_digitperm<float2>(in, out, dp);
+int digitperm(const qs_state* in, qs_state* out, const DigitList& list) {
+    return in->dtype == QS_C128 ? launch_digitperm<double2>(in, out, list)
+                                : launch_digitperm<float2>(in, out, list);
 }
 
 template <typename T>
-int launch_ket_pt(const qs_state* in, qs_state* out, const KetPT& p) {
-    hipLaunchKernelGGL(k_ket_pt<T>, dim3(grid_for(out->nelem, 256)), dim3(256), 0,
-                       in->stream, static_cast<const T*>(in->d),
-                       static_cast<T*>(out->d), p);
+int launch_ket_pt(const qs_state* in, qs_state* out, const DigitList& swapped) {
+    const uint64_t D = in->D;
+    const dim3 g(static_cast<uint32_t>((D + 255) / 256),
+                 static_cast<uint32_t>(std::min<uint64_t>(65535, (D + kPtCols - 1) / kPtCols)));
+    const T* src = static_cast<const T*>(in->d);
+    T* dst = static_cast<T*>(out->d);
+    Digits fit;
+    if (in->qubits) {
+        BitDigits bits{0};
+        for (const auto& d : swapped) bits.mask |= d.second;
+        hipLaunchKernelGGL((k_ket_pt<T, BitDigits>), g, dim3(256), 0, in->stream, src, dst, D, bits);
+    } else if (digits_fit(swapped, &fit))
+        hipLaunchKernelGGL((k_ket_pt<T, Digits>), g, dim3(256), 0, in->stream, src, dst, D, fit);
+    else
+        hipLaunchKernelGGL((k_ket_pt<T, WideDigits>), g, dim3(256), 0, in->stream, src, dst, D,
+                           wide_digits(swapped));
     QS_HIP(hipGetLastError(), "qpp_amd::ptranspose");
     return QS_OK;
 }
@@ -414,17 +423,11 @@ int qs_ptranspose(const qs_state* st, uint32_t ntarget, const uint64_t* target,
     }
     if (int rc = make_out(st, QS_RHO, st->dims, out)) return rc;
     if (st->kind == QS_KET) {
-        KetPT p{};
-        p.n = static_cast<uint32_t>(n);
-        p.D = st->D;
         if (n > 40) return fail(QS_ERR_NOT_IMPLEMENTED, W, "subsystems");
-        for (uint64_t q = 0; q < n; ++q) {
-            p.dim[q] = st->dims[q];
-            p.stride[q] = row_stride(st, q);
-            p.swap[q] = sw[q];
-        }
-        return st->dtype == QS_C128 ? launch_ket_pt<double2>(st, *out, p)
-                                    : launch_ket_pt<float2>(st, *out, p);
+        DigitList swapped;  // every digit, the others adding nothing
+        for (uint64_t q = 0; q < n; ++q) swapped.emplace_back(st->dims[q], sw[q] ? row_stride(st, q) : 0);
+        return st->dtype == QS_C128 ? launch_ket_pt<double2>(st, *out, swapped)
+                                    : launch_ket_pt<float2>(st, *out, swapped);
     }
     if (st->qubits) {
         std::vector<uint32_t> src(2 * n);
@@ -435,17 +438,12 @@ int qs_ptranspose(const qs_state* st, uint32_t ntarget, const uint64_t* target,
         }
         return bitperm(st, *out, src);
     }
-    DigitPerm dp{};
-    dp.nd = static_cast<uint32_t>(2 * n);
-    if (dp.nd > 80) return fail(QS_ERR_NOT_IMPLEMENTED, W, "subsystems");
+    if (2 * n > 80) return fail(QS_ERR_NOT_IMPLEMENTED, W, "subsystems");
     // output digits: column digits (most significant) then row digits
-    for (uint64_t q = 0; q < n; ++q) {
-        const uint64_t rs = row_stride(st, q), cs = rs * st->D;
-        dp.odim[q] = st->dims[q];
-        dp.istr[q] = sw[q] ? rs : cs;
-        dp.odim[n + q] = st->dims[q];
-        dp.istr[n + q] = sw[q] ? cs : rs;
-    }
+    DigitList dp;
+    for (int cols = 1; cols >= 0; --cols)
+        for (uint64_t q = 0; q < n; ++q)
+            dp.emplace_back(st->dims[q], row_stride(st, q) * ((cols != 0) != sw[q] ? st->D : 1));
     return digitperm(st, *out, dp);
 }
 
@@ -490,17 +488,10 @@ int qs_syspermute(const qs_state* st, const uint64_t* perm, qs_semantics sem,
     std::vector<uint64_t> odims(n);
     for (uint64_t k = 0; k < n; ++k) odims[k] = st->dims[pv[k]];
     if (int rc = make_out(st, st->kind, odims, out)) return rc;
-    DigitPerm dp{};
-    dp.nd = static_cast<uint32_t>(rho ? 2 * n : n);
-    if (dp.nd > 80) return fail(QS_ERR_NOT_IMPLEMENTED, W, "subsystems");
-    for (uint64_t k = 0; k < n; ++k) {
-        dp.odim[k + (rho ? n : 0)] = odims[k];
-        dp.istr[k + (rho ? n : 0)] = row_stride(st, pv[k]);
-        if (rho) {
-            dp.odim[k] = odims[k];
-            dp.istr[k] = row_stride(st, pv[k]) * st->D;
-        }
-    }
+    if ((rho ? 2 * n : n) > 80) return fail(QS_ERR_NOT_IMPLEMENTED, W, "subsystems");
+    DigitList dp;  // column digits (most significant), then row digits
+    for (int cols = rho ? 1 : 0; cols >= 0; --cols)
+        for (uint64_t k = 0; k < n; ++k) dp.emplace_back(odims[k], row_stride(st, pv[k]) * (cols ? st->D : 1));
     return digitperm(st, *out, dp);
 }
 

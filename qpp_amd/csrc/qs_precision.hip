@@ -191,7 +191,7 @@ int qs_state_convert(const qs_state* st, qs_dtype dtype, qs_state** out) {
     qs_state* r = nullptr;
     {
         const qs::StreamScope on(st->stream);
-        if (int rc = qs_state_create(dtype, st->kind, static_cast<uint32_t>(st->dims.size()),
+        if (int rc = qs::create_uninit(dtype, st->kind, static_cast<uint32_t>(st->dims.size()),
                                      st->dims.data(), &r))
             return rc;
     }

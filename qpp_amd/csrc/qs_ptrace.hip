@@ -14,47 +14,14 @@
 #include <cmath>
 #include <vector>
 
+#include "qs_digits.hpp"
 #include "qs_internal.hpp"
 
 namespace {
 
+using namespace qs_digits;
+
 typedef double doublex4 __attribute__((ext_vector_type(4)));
-
-// Mixed-radix digits, the last one fastest.  mag[k] = 2^32 / dim[k] rounded
-// up makes umulhi(v, mag) = v / dim exact while v * dim < 2^32, which the
-// host checks (digits_fit); dimensions of 1 are left out.
-constexpr int kMaxDigits = 40;
-struct Digits {
-    using Index = uint32_t;
-    uint32_t n;
-    uint32_t dim[kMaxDigits], mag[kMaxDigits];
-    uint64_t str[kMaxDigits];
-};
-// the same for any dimensions, by 64-bit division
-struct WideDigits {
-    using Index = uint64_t;
-    uint32_t n;
-    uint64_t dim[kMaxDigits], str[kMaxDigits];
-};
-
-__device__ __forceinline__ uint64_t offset_of(const Digits& g, uint32_t v) {
-    uint64_t off = 0;
-    for (int k = int(g.n) - 1; k >= 0; --k) {
-        const uint32_t q = __umulhi(v, g.mag[k]);
-        off += uint64_t(v - q * g.dim[k]) * g.str[k];
-        v = q;
-    }
-    return off;
-}
-
-__device__ __forceinline__ uint64_t offset_of(const WideDigits& g, uint64_t v) {
-    uint64_t off = 0;
-    for (int k = int(g.n) - 1; k >= 0; --k) {
-        off += (v % g.dim[k]) * g.str[k];
-        v /= g.dim[k];
-    }
-    return off;
-}
 
 // ---------------------------------------------------------------------------
 // kets: M M^dagger on the FP64 matrix cores
@@ -414,27 +381,6 @@ __global__ __launch_bounds__(256) void k_ptrace(const T* __restrict__ a, T* __re
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-using DigitList = std::vector<std::pair<uint64_t, uint64_t>>;  // (dim, stride)
-
-// false where a digit, their number or their product is out of reach of the
-// 32-bit quotients
-bool digits_fit(const DigitList& list, Digits* g) {
-    g->n = 0;
-    uint64_t count = 1;
-    for (const auto& [dim, str] : list) {
-        if (dim == 1) continue;
-        if (g->n == kMaxDigits || dim >= (uint64_t{1} << 32) || count >= (uint64_t{1} << 32) / dim)
-            return false;
-        count *= dim;
-        g->dim[g->n] = static_cast<uint32_t>(dim);
-        g->mag[g->n] = static_cast<uint32_t>(((uint64_t{1} << 32) + dim - 1) / dim);
-        g->str[g->n++] = str;
-    }
-    for (uint32_t k = 0; k < g->n; ++k)
-        if (count * g->dim[k] > (uint64_t{1} << 32)) return false;
-    return true;
-}
-
 uint64_t count_of(const DigitList& list) {
     uint64_t c = 1;
     for (const auto& d : list) c *= d.first;
@@ -549,11 +495,8 @@ int ptrace_impl(const qs_state* in, qs_state* out, const DigitList& keep, const 
         hipLaunchKernelGGL((k_ptrace<T, Digits>), g, dim3(256), 0, in->stream, src, dst, dk, dt, Dbar,
                            Dsub, in->D, sl, int(rho));
     } else {
-        WideDigits wk{}, wt{};
-        for (const auto& [dim, str] : keep) wk.dim[wk.n] = dim, wk.str[wk.n++] = str;
-        for (const auto& [dim, str] : ts) wt.dim[wt.n] = dim, wt.str[wt.n++] = str;
-        hipLaunchKernelGGL((k_ptrace<T, WideDigits>), g, dim3(256), 0, in->stream, src, dst, wk, wt,
-                           Dbar, Dsub, in->D, sl, int(rho));
+        hipLaunchKernelGGL((k_ptrace<T, WideDigits>), g, dim3(256), 0, in->stream, src, dst,
+                           wide_digits(keep), wide_digits(ts), Dbar, Dsub, in->D, sl, int(rho));
     }
     QS_HIP(hipGetLastError(), W);
     return QS_OK;
