@@ -161,34 +161,36 @@ bool is_diag(const std::vector<C>& m) {
     return m.size() == 4 && m[1] == C(0, 0) && m[2] == C(0, 0);
 }
 
-// Greedy capacity scheduling: walks `items` in order and takes every item
-// whose bits fit (with the bits already taken) into `cap` bits and that does
-// not touch a blocked qubit; items that do not fit block all their qubits so
-// later items on them keep their order.  Returns the indices taken.
-struct Item {
-    std::vector<uint32_t> need;   // bits that must be in the set
-    std::vector<uint32_t> touch;  // every bit the item depends on
+// A scheduling item: the bits that must be in the set, and every bit the
+// item depends on (which holds the former), as masks.
+struct Items {
+    std::vector<uint64_t> need, touch;
+    uint64_t all = 0;  // every bit an item touches
 };
 
-std::vector<size_t> greedy(const std::vector<Item>& items, const std::vector<size_t>& todo,
-                           std::set<uint32_t>& taken, size_t cap, size_t max_take) {
-    std::set<uint32_t> blocked;
+// Greedy capacity scheduling: walks `items` in order and takes every item
+// whose bits fit (with the bits already taken) into `cap` bits and that does
+// not touch a blocked bit; items that do not fit block all their bits so
+// later items on them keep their order.  Returns the indices taken.  Once
+// every bit is blocked, or max_take reached, no later item can be taken: a
+// random circuit's pass is decided by its next few layers, not by all that
+// is left of it.
+std::vector<size_t> greedy(const Items& items, const std::vector<size_t>& todo, uint64_t& taken, int cap,
+                           size_t max_take) {
+    uint64_t blocked = 0;
     std::vector<size_t> out;
     for (size_t id : todo) {
-        const Item& it = items[id];
-        bool blk = false;
-        for (uint32_t b : it.touch)
-            if (blocked.count(b)) blk = true;
-        if (!blk && out.size() < max_take) {
-            std::set<uint32_t> u = taken;
-            for (uint32_t b : it.need) u.insert(b);
-            if (u.size() <= cap) {
+        if (!(items.touch[id] & blocked)) {
+            const uint64_t u = taken | items.need[id];
+            if (__builtin_popcountll(u) <= cap) {
                 taken = u;
                 out.push_back(id);
+                if (out.size() == max_take) break;
                 continue;
             }
         }
-        for (uint32_t b : it.touch) blocked.insert(b);
+        blocked |= items.touch[id];
+        if (blocked == items.all) break;
     }
     return out;
 }
@@ -196,16 +198,16 @@ std::vector<size_t> greedy(const std::vector<Item>& items, const std::vector<siz
 // The gates a pass over the fixed tile-bit set S (a bit mask) takes: in
 // order, every gate whose needed bits lie in S and that touches no blocked
 // bit; a gate that cannot be taken blocks every bit it touches.
-size_t take_count(const std::vector<uint64_t>& need, const std::vector<uint64_t>& touch,
-                  const std::vector<size_t>& todo, uint64_t S, size_t max_take) {
+size_t take_count(const Items& items, const std::vector<size_t>& todo, uint64_t S, size_t max_take) {
     uint64_t blocked = 0;
     size_t n = 0;
     for (size_t id : todo) {
-        if (!(touch[id] & blocked) && !(need[id] & ~S) && n < max_take) {
-            ++n;
+        if (!(items.touch[id] & blocked) && !(items.need[id] & ~S)) {
+            if (++n == max_take) break;
             continue;
         }
-        blocked |= touch[id];
+        blocked |= items.touch[id];
+        if (blocked == items.all) break;
     }
     return n;
 }
@@ -213,10 +215,9 @@ size_t take_count(const std::vector<uint64_t>& need, const std::vector<uint64_t>
 // Improves a pass's tile-bit set by hill climbing: swap one of its free bits
 // (not among the `fixed` low bits) for a bit outside it while that lets the
 // pass take more gates.
-uint64_t improve_set(const std::vector<uint64_t>& need, const std::vector<uint64_t>& touch,
-                     const std::vector<size_t>& todo, uint64_t S, uint64_t fixed, uint32_t nb,
+uint64_t improve_set(const Items& items, const std::vector<size_t>& todo, uint64_t S, uint64_t fixed, uint32_t nb,
                      size_t max_take) {
-    size_t best = take_count(need, touch, todo, S, max_take);
+    size_t best = take_count(items, todo, S, max_take);
     for (bool improved = true; improved && best < max_take;) {
         improved = false;
         for (uint32_t b = 0; b < nb && !improved; ++b) {
@@ -224,7 +225,7 @@ uint64_t improve_set(const std::vector<uint64_t>& need, const std::vector<uint64
             for (uint32_t c = 0; c < nb && !improved; ++c) {
                 if ((S >> c) & 1) continue;
                 const uint64_t S2 = (S & ~(uint64_t{1} << b)) | (uint64_t{1} << c);
-                const size_t v = take_count(need, touch, todo, S2, max_take);
+                const size_t v = take_count(items, todo, S2, max_take);
                 if (v > best) {
                     best = v;
                     S = S2;
@@ -234,6 +235,32 @@ uint64_t improve_set(const std::vector<uint64_t>& need, const std::vector<uint64
         }
     }
     return S;
+}
+
+std::vector<uint32_t> bits_in(uint64_t mask) {
+    std::vector<uint32_t> v;
+    for (; mask; mask &= mask - 1) v.push_back(static_cast<uint32_t>(__builtin_ctzll(mask)));
+    return v;
+}
+
+uint64_t mask_of(const std::vector<uint32_t>& bits) {
+    uint64_t m = 0;
+    for (uint32_t b : bits) m |= uint64_t{1} << b;
+    return m;
+}
+
+// what is left of `todo` without the (ascending, in todo's order) `take`
+std::vector<size_t> without(const std::vector<size_t>& todo, const std::vector<size_t>& take) {
+    std::vector<size_t> rem;
+    rem.reserve(todo.size() - take.size());
+    size_t k = 0;
+    for (size_t i : todo) {
+        if (k < take.size() && take[k] == i)
+            ++k;
+        else
+            rem.push_back(i);
+    }
+    return rem;
 }
 
 // Layout of a phase: register tile bits R (ascending; register bit k is
@@ -319,28 +346,29 @@ FOp lower_op(const BitGate& g, const FPhase& ph, uint32_t RB, const std::vector<
              std::vector<C>& mats) {
     FOp op{};
     // where each global bit of the tile lives in this layout
-    std::map<uint32_t, int> reg_of, thr_of;
+    int reg_of[64], thr_of[64];  // -1: not there
+    std::fill(reg_of, reg_of + 64, -1);
+    std::fill(thr_of, thr_of + 64, -1);
     for (uint32_t k = 0; k < RB; ++k) reg_of[Sv[ph.regbits[k]]] = static_cast<int>(k);
     for (uint32_t j = 0; j < 8; ++j) thr_of[Sv[ph.tbits[j]]] = static_cast<int>(j);
     const uint32_t NR = 1u << RB;
     // control split
-    uint32_t regok = 0;
-    for (uint32_t rho = 0; rho < NR; ++rho) {
-        bool ok = true;
-        for (auto& kv : reg_of) {
-            const uint64_t bit = uint64_t{1} << kv.first;
-            if (!(g.cmask & bit)) continue;
-            const bool want = (g.cval & bit) != 0;
-            if ((((rho >> kv.second) & 1) != 0) != want) ok = false;
-        }
-        if (ok) regok |= 1u << rho;
-    }
-    op.regok = regok;
-    for (auto& kv : thr_of) {
-        const uint64_t bit = uint64_t{1} << kv.first;
+    uint32_t rmask = 0, rval = 0;  // the controls among the register bits
+    for (uint32_t k = 0; k < RB; ++k) {
+        const uint64_t bit = uint64_t{1} << Sv[ph.regbits[k]];
         if (!(g.cmask & bit)) continue;
-        op.tmask |= 1u << kv.second;
-        if (g.cval & bit) op.tval |= 1u << kv.second;
+        rmask |= 1u << k;
+        if (g.cval & bit) rval |= 1u << k;
+    }
+    uint32_t regok = 0;
+    for (uint32_t rho = 0; rho < NR; ++rho)
+        if ((rho & rmask) == rval) regok |= 1u << rho;
+    op.regok = regok;
+    for (uint32_t j = 0; j < 8; ++j) {
+        const uint64_t bit = uint64_t{1} << Sv[ph.tbits[j]];
+        if (!(g.cmask & bit)) continue;
+        op.tmask |= 1u << j;
+        if (g.cval & bit) op.tval |= 1u << j;
     }
     uint64_t in_tile = 0;
     for (uint32_t s : Sv) in_tile |= uint64_t{1} << s;
@@ -355,10 +383,10 @@ FOp lower_op(const BitGate& g, const FPhase& ph, uint32_t RB, const std::vector<
         const uint32_t b = g.bits[0];
         put(0, g.m[0]);
         put(1, g.m[3]);
-        if (reg_of.count(b)) {
+        if (reg_of[b] >= 0) {
             op.kind = OP_DIAG_R;
             op.j0 = reg_of[b];
-        } else if (thr_of.count(b)) {
+        } else if (thr_of[b] >= 0) {
             op.kind = OP_DIAG_T;
             op.tbit = 1u << thr_of[b];
         } else {
@@ -366,7 +394,7 @@ FOp lower_op(const BitGate& g, const FPhase& ph, uint32_t RB, const std::vector<
             op.dbit = uint64_t{1} << b;
         }
     } else if (g.bits.size() == 1) {
-        op.j0 = reg_of.at(g.bits[0]);
+        op.j0 = reg_of[g.bits[0]];
         if (is_x(g.m)) {
             op.kind = OP_X;
         } else {
@@ -375,7 +403,7 @@ FOp lower_op(const BitGate& g, const FPhase& ph, uint32_t RB, const std::vector<
         }
     } else {
         // bits[0] is the MSB of the gate index; kernel: LSB on j0 < j1
-        const int r0 = reg_of.at(g.bits[0]), r1 = reg_of.at(g.bits[1]);
+        const int r0 = reg_of[g.bits[0]], r1 = reg_of[g.bits[1]];
         op.kind = OP_U2;
         op.moff = static_cast<uint32_t>(mats.size());
         std::vector<C> mm = g.m;
@@ -468,52 +496,43 @@ int fused_compile(const std::vector<BitGate>& gates, uint32_t nb, const FusedOpt
     const uint32_t lc = std::min<uint32_t>(L, 2);
     // scheduling items: the bits a gate needs in the tile (none for a
     // diagonal 1-bit gate) and every bit it depends on
-    std::vector<Item> items(gates.size());
+    Items items;
+    items.need.resize(gates.size());
+    items.touch.resize(gates.size());
     for (size_t i = 0; i < gates.size(); ++i) {
         const BitGate& g = gates[i];
-        Item& it = items[i];
         const bool diag = g.bits.size() == 1 && is_diag(g.m);
-        if (!diag) it.need = g.bits;
-        it.touch = g.bits;
-        for (uint32_t b = 0; b < 64; ++b)
-            if ((g.cmask >> b) & 1) it.touch.push_back(b);
+        const uint64_t bits = mask_of(g.bits);
+        items.need[i] = diag ? 0 : bits;
+        items.touch[i] = bits | g.cmask;
+        items.all |= items.touch[i];
     }
     std::vector<size_t> todo(gates.size());
     for (size_t i = 0; i < todo.size(); ++i) todo[i] = i;
     P.gate_op.assign(gates.size(), -1);
-    std::vector<uint64_t> need_m(items.size()), touch_m(items.size());
-    for (size_t i = 0; i < items.size(); ++i) {
-        for (uint32_t b : items[i].need) need_m[i] |= uint64_t{1} << b;
-        for (uint32_t b : items[i].touch) touch_m[i] |= uint64_t{1} << b;
-    }
     const uint64_t low_mask = L >= 64 ? ~uint64_t{0} : (uint64_t{1} << L) - 1;
     std::vector<C> mats;
     while (!todo.empty()) {
-        std::set<uint32_t> S;
-        for (uint32_t b = 0; b < L; ++b) S.insert(b);
-        std::vector<size_t> take = greedy(items, todo, S, m, opt.max_ops);
+        uint64_t S = low_mask;
+        std::vector<size_t> take = greedy(items, todo, S, int(m), opt.max_ops);
         if (take.empty()) return fail(QS_ERR_NOT_IMPLEMENTED, "qpp_amd::fused", "gate wider than a tile");
         // fill S up to m bits with the lowest unused bits
-        for (uint32_t b = 0; S.size() < m && b < nb; ++b) S.insert(b);
+        for (uint32_t b = 0; __builtin_popcountll(S) < int(m) && b < nb; ++b) S |= uint64_t{1} << b;
         if (opt.improve_sets) {
-            uint64_t Sm = 0;
-            for (uint32_t b : S) Sm |= uint64_t{1} << b;
-            const uint64_t S2 = improve_set(need_m, touch_m, todo, Sm, low_mask, nb, opt.max_ops);
-            if (S2 != Sm) {
-                S.clear();
-                for (uint32_t b = 0; b < nb; ++b)
-                    if ((S2 >> b) & 1) S.insert(b);
-                std::set<uint32_t> full = S;
-                take = greedy(items, todo, full, m, opt.max_ops);
+            const uint64_t S2 = improve_set(items, todo, S, low_mask, nb, opt.max_ops);
+            if (S2 != S) {
+                S = S2;
+                uint64_t full = S;
+                take = greedy(items, todo, full, int(m), opt.max_ops);
             }
         }
         FPass ps{};
         ps.m = static_cast<int>(m);
-        std::vector<uint32_t> Sv(S.begin(), S.end());
+        const std::vector<uint32_t> Sv = bits_in(S);
         for (uint32_t i = 0; i < m; ++i) ps.S[i] = static_cast<uint8_t>(Sv[i]);
         std::vector<uint32_t> rest;
         for (uint32_t b = 0; b < nb; ++b)
-            if (!S.count(b)) rest.push_back(b);
+            if (!((S >> b) & 1)) rest.push_back(b);
         ps.nrest = static_cast<int>(rest.size());
         for (size_t i = 0; i < rest.size(); ++i) ps.rest[i] = static_cast<uint8_t>(rest[i]);
         ps.nruns = 0;
@@ -528,11 +547,13 @@ int fused_compile(const std::vector<BitGate>& gates, uint32_t nb, const FusedOpt
             return static_cast<uint32_t>(std::find(Sv.begin(), Sv.end(), g) - Sv.begin());
         };
         // phases: greedy over the pass's gates with capacity RB register bits
-        std::vector<Item> pit(take.size());
-        for (size_t i = 0; i < take.size(); ++i) {
-            const Item& it = items[take[i]];
-            for (uint32_t b : it.need) pit[i].need.push_back(tile_bit(b));
-            pit[i].touch = it.touch;  // dependencies on global bits
+        Items pit;
+        for (size_t id : take) {
+            uint64_t need = 0;
+            for (uint32_t b : bits_in(items.need[id])) need |= uint64_t{1} << tile_bit(b);
+            pit.need.push_back(need);
+            pit.touch.push_back(items.touch[id]);  // dependencies on global bits
+            pit.all |= items.touch[id];
         }
         std::vector<size_t> ptodo(take.size());
         for (size_t i = 0; i < ptodo.size(); ++i) ptodo[i] = i;
@@ -543,23 +564,16 @@ int fused_compile(const std::vector<BitGate>& gates, uint32_t nb, const FusedOpt
         // load phase (top RB tile bits, no ops) comes first and the kernel
         // returns to it before storing.
         bool first = true;
-        std::vector<uint64_t> pneed(pit.size()), ptouch(pit.size());
-        for (size_t i = 0; i < pit.size(); ++i) {
-            for (uint32_t b : pit[i].need) pneed[i] |= uint64_t{1} << b;
-            for (uint32_t b : pit[i].touch) ptouch[i] |= uint64_t{1} << b;
-        }
         while (!ptodo.empty()) {
-            std::set<uint32_t> R;
-            std::vector<size_t> ptake = greedy(pit, ptodo, R, RB, SIZE_MAX);
-            // complete R with unused tile bits, preferring high ones
-            for (int b = int(m) - 1; R.size() < RB && b >= 0; --b) R.insert(uint32_t(b));
+            uint64_t Rm = 0;
+            std::vector<size_t> ptake = greedy(pit, ptodo, Rm, int(RB), SIZE_MAX);
+            // complete the register bits with unused tile bits, preferring high ones
+            for (int b = int(m) - 1; __builtin_popcountll(Rm) < int(RB) && b >= 0; --b) Rm |= uint64_t{1} << b;
             if (opt.improve_sets) {
                 // hill climbing on the register bits, as for the passes' tile
                 // bits: swap one for another tile bit while the phase then
                 // takes more gates (tile bits below lc stay out, so a
                 // coalesced phase stays coalesced)
-                uint64_t Rm = 0;
-                for (uint32_t b : R) Rm |= uint64_t{1} << b;
                 // gates taken, then (on ties) gates on tile bits below lc
                 // taken: a phase that does them early leaves a coalesced
                 // layout for the pass's store more often
@@ -568,12 +582,13 @@ int fused_compile(const std::vector<BitGate>& gates, uint32_t nb, const FusedOpt
                     uint64_t blocked = 0;
                     size_t n = 0, low = 0;
                     for (size_t id : ptodo) {
-                        if (!(ptouch[id] & blocked) && !(pneed[id] & ~Rx)) {
+                        if (!(pit.touch[id] & blocked) && !(pit.need[id] & ~Rx)) {
                             ++n;
-                            if (pneed[id] & lowm) ++low;
+                            if (pit.need[id] & lowm) ++low;
                             continue;
                         }
-                        blocked |= ptouch[id];
+                        blocked |= pit.touch[id];
+                        if (blocked == pit.all) break;
                     }
                     return n * 1024 + low;
                 };
@@ -596,12 +611,11 @@ int fused_compile(const std::vector<BitGate>& gates, uint32_t nb, const FusedOpt
                         }
                     }
                 }
-                R.clear();
-                for (uint32_t b = 0; b < m; ++b)
-                    if ((Rm >> b) & 1) R.insert(b);
-                std::set<uint32_t> Rg = R;
-                ptake = greedy(pit, ptodo, Rg, RB, SIZE_MAX);
+                uint64_t Rg = Rm;
+                ptake = greedy(pit, ptodo, Rg, int(RB), SIZE_MAX);
             }
+            std::set<uint32_t> R;
+            for (uint32_t b : bits_in(Rm)) R.insert(b);
             const FPhase* prev = first ? nullptr : &P.phases.back();
             FPhase ph = make_phase(R, m, RB, Sv, lc, prev);
             if (first && !ph.coalesced) {
@@ -619,21 +633,13 @@ int fused_compile(const std::vector<BitGate>& gates, uint32_t nb, const FusedOpt
             ph.op_end = static_cast<int>(P.ops.size());
             if (opt.bundle) bundle_phase(P, ph, RB, mats);
             P.phases.push_back(ph);
-            std::vector<size_t> rem;
-            std::set<size_t> tk(ptake.begin(), ptake.end());
-            for (size_t i : ptodo)
-                if (!tk.count(i)) rem.push_back(i);
-            ptodo.swap(rem);
+            ptodo = without(ptodo, ptake);
             first = false;
         }
         ps.phase_end = static_cast<int>(P.phases.size());
         P.passes.push_back(ps);
         P.gates_per_pass.push_back(take.size());
-        std::vector<size_t> rem;
-        std::set<size_t> tk(take.begin(), take.end());
-        for (size_t i : todo)
-            if (!tk.count(i)) rem.push_back(i);
-        todo.swap(rem);
+        todo = without(todo, take);
     }
     P.mats = mats;
     P.reg_bits = RB;
