@@ -714,7 +714,8 @@ __global__ __launch_bounds__(256) void k_put(uint32_t* __restrict__ d, PutChunk 
 
 // Device copy of a host table of one call (matrices, offsets), a multiple of
 // 4 bytes.  Up to kTabBytes it goes into the state's own table memory, which
-// its next call overwrites in stream order: a few launches, where an
+// its next call overwrites in stream order (the caller holds tab_mutex until
+// the kernel that reads it is launched): a few launches, where an
 // allocation, a pageable copy, its wait and the free took 25 us (16 KiB: six
 // launches).  Larger tables are copied into memory of their own (*owned),
 // freed stream-ordered after the kernel.
@@ -813,6 +814,7 @@ int gate_reg(qs_state* st, const uint32_t* regs, const double* m, bool conj, con
     } else {
         cxt<R> mm[DIM * DIM];
         for (int i = 0; i < DIM * DIM; ++i) mm[i] = to_c<R>(m, i, conj);
+        const std::lock_guard<std::mutex> hold(st->tab_mutex);
         void *d = nullptr, *owned = nullptr;
         static_assert(sizeof(mm) <= kTabBytes, "in the state's table memory");
         if (int rc = upload(st, mm, sizeof(mm), &d, &owned)) return rc;
@@ -857,6 +859,7 @@ int gatek_impl(qs_state* st, const uint32_t* bits, uint32_t k, const double* m,
     std::vector<unsigned char> blob(inner_bytes + mat_bytes);
     std::memcpy(blob.data(), inner.data(), inner_bytes);
     std::memcpy(blob.data() + inner_bytes, mm.data(), mat_bytes);
+    const std::lock_guard<std::mutex> hold(st->tab_mutex);
     void *dblob = nullptr, *owned = nullptr;
     if (int rc = upload(st, blob.data(), blob.size(), &dblob, &owned)) return rc;
     constexpr int EPT = 4;
@@ -908,6 +911,7 @@ int gatek_mfma(qs_state* st, uint32_t k, const std::vector<uint64_t>& inner, con
     QS_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), "qpp::apply()");
     const uint32_t resident = static_cast<uint32_t>(std::max(1, per_cu) * std::max(1, ncu));
     const uint32_t grid = std::min<uint32_t>(grid_for(groups16, kBlock / 64), std::min(kMfmaGrid, resident));
+    const std::lock_guard<std::mutex> hold(st->tab_mutex);
     void *dblob = nullptr, *owned = nullptr;
     if (int rc = upload(st, blob.data(), blob.size(), &dblob, &owned)) return rc;
     auto* inn = static_cast<const uint64_t*>(dblob);
@@ -949,6 +953,7 @@ int qudit_reg(qs_state* st, const qs::QuditGate& g, const std::vector<uint64_t>&
             hipLaunchKernelGGL(by_value, grid, dim3(kBlock), 0, st->stream, a, ns, f, m);
             return QS_OK;
         }
+        const std::lock_guard<std::mutex> hold(st->tab_mutex);
         void *d = nullptr, *owned = nullptr;
         if (int rc = upload(st, mm.data(), mm.size() * sizeof(cxt<R>), &d, &owned)) return rc;
         GateMatN<R, kQuditMats, false> m;
@@ -1012,6 +1017,7 @@ int qudit_impl(qs_state* st, const qs::QuditGate& g, const double* mats,
     std::vector<unsigned char> blob(off_bytes + mat_bytes);
     std::memcpy(blob.data(), off.data(), off_bytes);
     std::memcpy(blob.data() + off_bytes, mm.data(), mat_bytes);
+    const std::lock_guard<std::mutex> hold(st->tab_mutex);
     void *dblob = nullptr, *owned = nullptr;
     if (int rc = upload(st, blob.data(), blob.size(), &dblob, &owned)) return rc;
     const auto* dmats = reinterpret_cast<const cxt<R>*>(static_cast<unsigned char*>(dblob) + off_bytes);

@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -31,7 +32,11 @@ struct qs_state {
     bool qubits = true;          // all dims == 2
     uint32_t nbits = 0;          // log2(nelem) when qubits
     void* d = nullptr;           // device buffer
-    void* tab = nullptr;         // small tables of the call in progress (qs_gates.hip), on first use
+    // small tables of the gate call in progress (qs_gates.hip), on first use;
+    // held from writing them to launching the kernel that reads them, so that
+    // calls of several threads on one state follow each other
+    void* tab = nullptr;
+    std::mutex tab_mutex;
     hipStream_t stream = nullptr;
     int device = 0;
     uint64_t elem_bytes() const { return dtype == QS_C128 ? 16 : 8; }

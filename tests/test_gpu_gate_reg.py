@@ -75,3 +75,29 @@ def test_rho_gates(qa, orc, n, dtype):
             st = qa.State.from_array(rho, [2] * n, dtype=dt)
             t = sets[-1]
             assert np.max(np.abs(st.apply_kraus(Ks, t).download() - orc.apply_kraus(rho, Ks, t, 2))) <= tol, t
+
+
+@pytest.mark.parametrize("k", [4, 5])
+def test_gates_from_two_threads(qa, k):
+    """Commuting (diagonal) gates applied to one state by two threads at once,
+    each call with a table of its own in device memory: the product of all,
+    whatever the order."""
+    import threading
+    n, reps = 10, 200
+    rng = np.random.default_rng(k)
+    psi = randket(2 ** n, rng)
+    phases = [np.exp(2j * np.pi * rng.random(2 ** k) / reps) for _ in range(2)]
+    st = qa.State.from_array(psi, [2] * n)
+    t = list(range(2, 2 + k))
+
+    def work(d):
+        for _ in range(reps):
+            st.apply(np.diag(d), t)
+
+    threads = [threading.Thread(target=work, args=(d,)) for d in phases]
+    for x in threads:
+        x.start()
+    for x in threads:
+        x.join()
+    want = psi.reshape(4, 2 ** k, -1) * ((phases[0] * phases[1]) ** reps)[None, :, None]
+    assert np.max(np.abs(st.download() - want.reshape(-1))) <= 1e-12  # 400 products of modulus 1
