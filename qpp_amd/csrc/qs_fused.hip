@@ -99,11 +99,11 @@ __global__ __launch_bounds__(kThreads) void k_tile(cxt<R>* __restrict__ a,
             const int ob = ph->op_begin, oe = ph->op_end;
             int o = ob;
             for (; o + 1 < oe; o += 2) {
-                run_op<R, NR>(x, z, ops + o, ops[o].m, mats, t, base);
-                run_op<R, NR>(z, x, ops + o + 1, ops[o + 1].m, mats, t, base);
+                run_op<R, NR, true>(x, z, ops + o, ops[o].m, mats, t, base);
+                run_op<R, NR, true>(z, x, ops + o + 1, ops[o + 1].m, mats, t, base);
             }
             if (o < oe) {
-                run_op<R, NR>(x, z, ops + o, ops[o].m, mats, t, base);
+                run_op<R, NR, true>(x, z, ops + o, ops[o].m, mats, t, base);
                 copy_regs<R, NR>(z, x);
             }
         }

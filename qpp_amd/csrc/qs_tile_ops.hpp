@@ -273,7 +273,7 @@ __device__ __forceinline__ void do_u2(const cxt<R>* x, cxt<R>* y, uint32_t regok
             break;                                                 \
     }
 
-template <typename R, int NR, bool CT>
+template <typename R, int NR, bool CT, bool SELECT>
 __device__ __forceinline__ void run_op_ct(const cxt<R>* x, cxt<R>* y, const OpHead& h,
                                           const FOp* op, const double* mu,
                                           const cxt<R>* mats, uint32_t t, uint64_t base,
@@ -301,7 +301,7 @@ __device__ __forceinline__ void run_op_ct(const cxt<R>* x, cxt<R>* y, const OpHe
             do_scale<R, NR, CT>(x, y, regok, d, tok);
             break;
         }
-        case OP_U1S: {
+        case OP_U1S: if constexpr (SELECT) {
             // U where the condition fails, the second matrix where it holds
             const cxt<R>* M = mats + h.moff;
             if constexpr (!CT) {  // a tile condition: uniform
@@ -312,10 +312,12 @@ __device__ __forceinline__ void run_op_ct(const cxt<R>* x, cxt<R>* y, const OpHe
             }
             break;
         }
+        copy_regs<R, NR>(x, y);
+        break;
         case OP_U2S:  // (tile conditions only)
         case OP_U2: {
             const cxt<R>* M = mats + h.moff;
-            if (!CT && (code & 15u) == OP_U2S && (base & op->omask) == op->oval) M += 16;
+            if (SELECT && !CT && (code & 15u) == OP_U2S && (base & op->omask) == op->oval) M += 16;
             switch (j0 * 4 + j1) {
                 case 0 * 4 + 1: do_u2<R, NR, 0, 1, CT>(x, y, regok, M, tok); break;
                 case 0 * 4 + 2: do_u2<R, NR, 0, 2, CT>(x, y, regok, M, tok); break;
@@ -346,7 +348,7 @@ __device__ __forceinline__ void run_op_ct(const cxt<R>* x, cxt<R>* y, const OpHe
 // the diagonal) the op applies: h.m, or a per-trajectory override of it.
 // Bundles, the commonest op, are never controlled and go first, on a path
 // that holds nothing but their arithmetic.
-template <typename R, int NR>
+template <typename R, int NR, bool SELECT>
 __device__ __forceinline__ void run_op_h(const cxt<R>* x, cxt<R>* y, const OpHead& h,
                                          const FOp* op, const double* mu, const cxt<R>* mats,
                                          uint32_t t, uint64_t base) {
@@ -361,9 +363,9 @@ __device__ __forceinline__ void run_op_h(const cxt<R>* x, cxt<R>* y, const OpHea
     }
     if (code & kCodeCtrl) {
         const bool tok = (t & h.tmask) == h.tval;
-        run_op_ct<R, NR, true>(x, y, h, op, mu, mats, t, base, tok);
+        run_op_ct<R, NR, true, SELECT>(x, y, h, op, mu, mats, t, base, tok);
     } else {
-        run_op_ct<R, NR, false>(x, y, h, op, mu, mats, t, base, true);
+        run_op_ct<R, NR, false, SELECT>(x, y, h, op, mu, mats, t, base, true);
     }
 }
 
@@ -371,13 +373,14 @@ __device__ __forceinline__ OpHead load_head(const FOp* op) {
     return *reinterpret_cast<const OpHead*>(op);
 }
 
-// y := op(x), loading the op's head here
-template <typename R, int NR>
+// y := op(x), loading the op's head here.  SELECT: pair-fused programs, with
+// OP_U1S and OP_U2S; without them the code is smaller (batches).
+template <typename R, int NR, bool SELECT = false>
 __device__ __forceinline__ void run_op(const cxt<R>* x, cxt<R>* y, const FOp* op,
                                        const double* mu, const cxt<R>* mats, uint32_t t,
                                        uint64_t base) {
     const OpHead h = load_head(op);
-    run_op_h<R, NR>(x, y, h, op, mu, mats, t, base);
+    run_op_h<R, NR, SELECT>(x, y, h, op, mu, mats, t, base);
 }
 
 // Global index bits of tile number `tile` (the pass's out-of-tile bits as
