@@ -33,7 +33,6 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <limits>
 #include <map>
 #include <mutex>
 #include <thread>
@@ -538,38 +537,6 @@ FusedProgram native_fuse(const FusedProgram& P) {
 
 namespace {
 
-// A 4x4 that keeps Hermitian matrices Hermitian (a superoperator on the row
-// and column bit of one qubit: U rho U^dagger, channels and their products)
-// is a real matrix R over the Pauli components of its four amplitudes,
-//   I = v0 + v3, Z = v0 - v3, X = v1 + v2, Y = i (v1 - v2):
-// M = T^-1 R T with 16 additions for T and T^-1 and two multiply-adds per
-// entry of R that is not zero, 36 FP64 instructions for four amplitudes of a
-// unital channel (three rows of three entries) and at most 48, where the
-// dense product takes 64.  Entries below rounding (the trace row, the unital
-// column) are dropped.  The passes of a 12-qubit density-matrix circuit with
-// depolarizing noise: 117 -> 101 us each, the error against 80-bit sums no
-// larger (1.8e-15 either way, complex64 3.9e-7 against 4.1e-7).
-bool pauli_form(const C* M, double (&R)[16]) {
-    const C i(0, 1);
-    const C T[4][4] = {{1, 0, 0, 1}, {1, 0, 0, -1}, {0, 1, 1, 0}, {0, i, -i, 0}};
-    double top = 0, imag = 0;
-    for (int r = 0; r < 4; ++r)
-        for (int c = 0; c < 4; ++c) {
-            C v(0, 0);  // (T M T^dagger)_rc / 2
-            for (int a = 0; a < 4; ++a)
-                for (int b = 0; b < 4; ++b) v += T[r][a] * M[a + 4 * b] * std::conj(T[c][b]);
-            v *= 0.5;
-            R[4 * r + c] = v.real();
-            top = std::max(top, std::abs(v));
-            imag = std::max(imag, std::abs(v.imag()));
-        }
-    const double tiny = 32 * std::numeric_limits<double>::epsilon() * top;
-    if (!(imag <= tiny)) return false;
-    for (double& v : R) v = std::abs(v) <= tiny ? 0.0 : v / 2;  // the 1/2 of T^-1
-    if (std::abs(R[0] - 0.5) <= tiny) R[0] = 0.5;  // trace kept
-    return true;
-}
-
 // y = op(x) for one op, in place on the register array under the current
 // renaming (qs_tile_ops.hpp run_op_h / run_op_ct / do_*)
 // fx: an X on one register bit under a lane or tile condition, folded into
@@ -772,42 +739,6 @@ void gen_op(Gen& g, const FusedProgram& P, const FOp& op, const FOp* fx = nullpt
                 for (int i = 0; i < 16; ++i)
                     o << (i ? ", " : "") << "mk(cm[" << i0 + 2 * i << " + so], cm[" << i0 + 2 * i + 1 << " + so])";
                 o << "};\n";
-            } else if (double R[16]; !fx && pauli_form(M, R)) {
-                std::string e[16];
-                for (int i = 0; i < 16; ++i)
-                    if (R[i] != 0.0) e[i] = "cm[" + std::to_string(g.tab.size()) + "]", (void)g.cx(R[i], 0.0);
-                const char* w[4] = {"wi", "wz", "wx", "wy"};
-                for (int rho = 0; rho < kNR; ++rho) {
-                    if (((rho >> J0) & 1) || ((rho >> J1) & 1)) continue;
-                    if (!rok(rho)) continue;
-                    const int i[4] = {rho, rho | (1 << J0), rho | (1 << J1), rho | (1 << J0) | (1 << J1)};
-                    o << "    { const T v0 = " << g.X(i[0]) << ", v1 = " << g.X(i[1]) << ", v2 = " << g.X(i[2])
-                      << ", v3 = " << g.X(i[3]) << ";\n"
-                      << "    const T wi = mk(v0.x + v3.x, v0.y + v3.y), wz = mk(v0.x - v3.x, v0.y - v3.y);\n"
-                      << "    const T wx = mk(v1.x + v2.x, v1.y + v2.y), wy = mk(v2.y - v1.y, v1.x - v2.x);\n";
-                    for (int r = 0; r < 4; ++r) {
-                        std::string part[2];
-                        for (int c = 0; c < 4; ++c) {
-                            if (e[4 * r + c].empty()) continue;
-                            for (int k = 0; k < 2; ++k)
-                                part[k] += (part[k].empty() ? "" : " + ") + e[4 * r + c] + " * " + w[c] + (k ? ".y" : ".x");
-                        }
-                        for (std::string& q : part)
-                            if (q.empty()) q = "R(0)";
-                        o << "    const T " << w[r] << "n = mk(" << part[0] << ", " << part[1] << ");\n";
-                    }
-                    const char* out[4] = {"mk(win.x + wzn.x, win.y + wzn.y)", "mk(wxn.x + wyn.y, wxn.y - wyn.x)",
-                                          "mk(wxn.x - wyn.y, wxn.y + wyn.x)", "mk(win.x - wzn.x, win.y - wzn.y)"};
-                    for (int r = 0; r < 4; ++r) {
-                        o << "    " << g.X(i[r]) << " = ";
-                        if (has_t)
-                            o << "sel(tk, " << out[r] << ", v" << r << ");\n";
-                        else
-                            o << out[r] << ";\n";
-                    }
-                    o << "    }\n";
-                }
-                break;
             } else {
                 o << "    const T m[16] = {";
                 for (int i = 0; i < 16; ++i) o << (i ? ", " : "") << g.cx(M[i]);

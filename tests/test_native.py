@@ -9,7 +9,7 @@ persistent workgroups walking many tiles, and at the benchmark's full size
 import numpy as np
 import pytest
 
-from helpers import randket, randrho
+from helpers import haar, randket, randrho
 from test_gpu_fused import maxabs, mixed_circuit, oracle_run
 
 pytestmark = pytest.mark.gpu
@@ -163,3 +163,121 @@ def test_native_sign_diagonals_vs_oracle(qa, orc):
         p.run(st)
         tol = TOL if dt == qa.C128 else 5e-6
         assert maxabs(st.download().astype(np.complex128), oracle_run(orc, psi, qc)) <= tol, (n, seed)
+
+
+def _channels(kind, p):
+    """(Kraus operators, the 2x2 map of the two populations) of a channel
+    that keeps populations apart from coherences."""
+    from qpp_amd import workloads
+    if kind == "damping":
+        return ([np.diag([1, np.sqrt(1 - p)]).astype(complex),
+                 np.array([[0, np.sqrt(p)], [0, 0]], dtype=complex)], [[1, p], [0, 1 - p]])
+    return workloads.depolarizing_kraus(p), [[1 - 2 * p / 3, 2 * p / 3], [2 * p / 3, 1 - 2 * p / 3]]
+
+
+@pytest.mark.parametrize("dtype", ["c128", "c64"])
+@pytest.mark.parametrize("channels", [[("damping", 0.01)], [("depolarizing", 1e-6)],
+                                      [("damping", 0.3), ("depolarizing", 1e-6), ("damping", 1e-4)]])
+def test_native_small_populations(qa, channels, dtype):
+    """Channels on a diagonal density matrix whose populations span 21 orders
+    of magnitude: every one is a sum of non-negative products, so it stays
+    non-negative and keeps its relative accuracy however small it is beside
+    the others.  The reference acts on the populations in extended precision;
+    per channel a superoperator entry is within 8 roundings of it (the Kraus
+    operators' roots, products and sum, in FP64, and its rounding to the
+    state's type), the 4-term product within 4."""
+    n = 6
+    dt, eps, ctype = (qa.C128, 2.0 ** -53, np.complex128) if dtype == "c128" else (qa.C64, 2.0 ** -24, np.complex64)
+    pops = np.ones(1, dtype=np.longdouble)
+    for q in range(n):
+        pops = np.kron(pops, np.array([1, 10.0 ** -(q + 1)], dtype=np.longdouble))
+    pops = np.real(pops.astype(ctype)).astype(np.longdouble)
+    bp = qa.BitProgram(2 * n)
+    ref = pops.reshape([2] * n)
+    for kind, p in channels:
+        for q in range(n):
+            Ks, M = _channels(kind, p)
+            bp.rho_channel(Ks, q, n)
+            ref = np.moveaxis(np.tensordot(np.array(M, dtype=np.longdouble), ref, axes=(1, q)), 0, q)
+    ref = ref.reshape(-1)
+    bp.compile(dtype=dt)
+    tol = 12 * eps * n * len(channels)
+    for native in (False, True):
+        st = qa.State.from_array(np.diag(pops.astype(ctype)), [2] * n, dtype=dt)
+        if native:
+            bp.compile_native()
+        bp.run(st)
+        got = np.asarray(st.download())
+        d = np.real(np.diag(got)).astype(np.longdouble)
+        assert d.min() >= 0, (native, d.min())
+        err = float(np.max(np.abs(d - ref) / ref))
+        print(f"small populations {channels} {dtype} native={native}: relative error {err:.2e}", flush=True)
+        assert err <= tol, (native, err, tol)
+        assert not np.any(got - np.diag(np.diag(got)))
+
+
+@pytest.mark.parametrize("dtype", ["c128", "c64"])
+def test_bit_program_superoperators_vs_oracle(qa, orc, dtype):
+    """Dense 4x4s of every kind a density-matrix program holds (depolarizing
+    and amplitude damping superoperators, which mix populations one way, SWAP
+    and Haar gates), some under controls that land on register, lane and
+    out-of-tile bits, against the oracle applied op by op: specialised
+    kernels, the tile kernel's fused program and its unfused one (reg_bits
+    3).  The superoperators are within a factor 2 of norm 1, so the error is
+    measured against the result's largest amplitude."""
+    nb = 14
+    rng = np.random.default_rng(77)
+    swap = np.eye(4)[[0, 2, 1, 3]].astype(complex)
+    bp, ops = qa.BitProgram(nb), []
+    for i in range(60):
+        bits = [int(b) for b in rng.permutation(nb)[:5]]
+        kind = i % 5
+        if kind < 2:
+            Ks, _ = _channels("damping" if kind else "depolarizing", 0.05)
+            M = sum(np.kron(K.conj(), K) for K in Ks)
+        else:
+            M = {2: swap, 3: haar(4, rng), 4: haar(2, rng)}[kind]
+        nt = 1 if kind == 4 else 2
+        ctrl = bits[2:2 + int(rng.integers(0, 4))]
+        shift = [int(s) for s in rng.integers(0, 2, len(ctrl))]
+        bp.gate(M, bits[:nt], sum(1 << c for c in ctrl), sum(1 << c for c, s in zip(ctrl, shift) if not s))
+        ops.append((M, [nb - 1 - b for b in bits[:nt]], [nb - 1 - c for c in ctrl], shift))
+    dt, tol = (qa.C128, 1e-12) if dtype == "c128" else (qa.C64, 1e-5)
+    psi = randket(2 ** nb, rng)
+    ref = psi
+    for M, t, c, shift in ops:
+        ref = orc.applyCTRL(ref, M, c, t, 2, shift) if c else orc.apply(ref, M, t, 2)
+    for name in ("unfused", "fused", "specialised"):
+        bp.compile(dtype=dt, reg_bits=3 if name == "unfused" else 4)
+        if name == "specialised":
+            bp.compile_native()
+        st = qa.State.from_array(psi, [2] * nb, dtype=dt)
+        bp.run(st)
+        err = maxabs(np.asarray(st.download()).astype(np.complex128), ref) / np.max(np.abs(ref))
+        print(f"superoperators {dtype} {name}: {err:.2e}", flush=True)
+        assert err <= tol, (name, err)
+
+
+@pytest.mark.parametrize("dtype", ["c128", "c64"])
+def test_native_rho_pipeline_vs_oracle(qa, orc, dtype):
+    """The density-matrix pipeline's circuit through the specialised and the
+    tile kernel against the oracle, gate by gate and channel by channel."""
+    from qpp_amd import workloads
+    n = 6
+    rho, ops, _, _, _ = workloads.dm_pipeline(n, 3, seed=5)
+    ref = rho
+    for kind, q, M in ops:
+        if kind == "kraus":
+            ref = orc.apply_kraus(ref, M, q, 2)
+        elif kind == "cz":
+            ref = orc.applyCTRL(ref, M, [q[0]], [q[1]], 2)
+        else:
+            ref = orc.apply(ref, M, q, 2)
+    dt, tol = (qa.C128, TOL) if dtype == "c128" else (qa.C64, 5e-6)
+    for native in (False, True):
+        p = workloads.dm_program(qa, n, ops).compile(dtype=dt)
+        if native:
+            p.compile_native()
+        st = qa.State.from_array(rho, [2] * n, dtype=dt)
+        p.run(st)
+        assert maxabs(np.asarray(st.download()).astype(np.complex128), ref) <= tol, native
