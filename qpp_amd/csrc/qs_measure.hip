@@ -151,8 +151,9 @@ __global__ __launch_bounds__(1024) void k_scan_chunks(const double* __restrict__
     if (threadIdx.x == 0) prefix[nchunks] = total;
 }
 
-// One wave per shot: binary search over chunk prefixes, then an in-chunk
-// wave scan.  Writes the candidate index and whether it is certain.
+// One wave per shot (a grid of waves over all shots): binary search over
+// chunk prefixes, then an in-chunk wave scan.  Writes the candidate index and
+// whether it is certain.
 __global__ __launch_bounds__(256) void k_search(const double* __restrict__ p,
                                                 uint64_t D,
                                                 const double* __restrict__ prefix,
@@ -161,60 +162,61 @@ __global__ __launch_bounds__(256) void k_search(const double* __restrict__ p,
                                                 uint64_t nshots, double B,
                                                 uint64_t* __restrict__ idx,
                                                 int* __restrict__ certain) {
-    const uint64_t wave = (uint64_t(blockIdx.x) * 256 + threadIdx.x) / 64;
+    const uint64_t nwaves = uint64_t(gridDim.x) * 4;
     const int lane = threadIdx.x & 63;
-    if (wave >= nshots) return;
     const double total = prefix[nchunks];
-    const double uu = u[wave];
-    const double target = uu * total;
-    // last chunk whose exclusive prefix is < target (chunk 0 if none)
-    uint64_t lo = 0, hi = nchunks;  // invariant: prefix[lo] < target or lo == 0
-    while (hi - lo > 1) {
-        const uint64_t mid = (lo + hi) / 2;
-        if (prefix[mid] < target)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    // the 64 elements of the chunk that hold the first E_k >= target: each
-    // lane sums 64 consecutive ones; then those, one a lane
-    const uint64_t b = lo * kChunk;
-    double v = 0;
-#pragma unroll 16
-    for (int j = 0; j < kChunk / 64; ++j) {
-        const uint64_t i = b + uint64_t(lane) * (kChunk / 64) + j;
-        v += i < D ? p[i] : 0.0;
-    }
-    const double inc = wave_incl_sum(v, lane);
-    unsigned long long hit = __ballot(prefix[lo] + inc >= target);
-    uint64_t found = D;  // D = not found in this chunk
-    double e_prev = 0, e_at = 0;
-    if (hit) {
-        const int l0 = __ffsll(hit) - 1;
-        const double run = prefix[lo] + (l0 ? __shfl(inc, l0 - 1, 64) : 0.0);
-        const uint64_t s = b + uint64_t(l0) * (kChunk / 64);
-        const uint64_t i = s + lane;
-        const double x = i < D ? p[i] : 0.0;
-        const double e = run + wave_incl_sum(x, lane);
-        hit = __ballot(i < D && e >= target);
-        if (hit) {  // (rounding may leave the last one below the target)
-            const int l = __ffsll(hit) - 1;
-            found = s + l;
-            e_at = __shfl(e, l, 64);
-            e_prev = __shfl(e - x, l, 64);
+    for (uint64_t shot = (uint64_t(blockIdx.x) * 256 + threadIdx.x) / 64; shot < nshots; shot += nwaves) {
+        const double uu = u[shot];
+        const double target = uu * total;
+        // last chunk whose exclusive prefix is < target (chunk 0 if none)
+        uint64_t lo = 0, hi = nchunks;  // invariant: prefix[lo] < target or lo == 0
+        while (hi - lo > 1) {
+            const uint64_t mid = (lo + hi) / 2;
+            if (prefix[mid] < target)
+                lo = mid;
+            else
+                hi = mid;
         }
-    }
-    if (lane == 0) {
-        if (found == D) {
-            // past the end of the chunk: the sequential table's last entry is
-            // forced to 1, so the answer is certain only away from the edge
-            idx[wave] = D - 1;
-            certain[wave] = 0;
-        } else {
-            idx[wave] = found;
-            const double lo_edge = e_prev / total, hi_edge = e_at / total;
-            certain[wave] = (lo_edge < uu - B) && (hi_edge >= uu + B) &&
-                            (found != D - 1 || hi_edge >= uu + B);
+        // the 64 elements of the chunk that hold the first E_k >= target: each
+        // lane sums 64 consecutive ones; then those, one a lane
+        const uint64_t b = lo * kChunk;
+        double v = 0;
+#pragma unroll 16
+        for (int j = 0; j < kChunk / 64; ++j) {
+            const uint64_t i = b + uint64_t(lane) * (kChunk / 64) + j;
+            v += i < D ? p[i] : 0.0;
+        }
+        const double inc = wave_incl_sum(v, lane);
+        unsigned long long hit = __ballot(prefix[lo] + inc >= target);
+        uint64_t found = D;  // D = not found in this chunk
+        double e_prev = 0, e_at = 0;
+        if (hit) {
+            const int l0 = __ffsll(hit) - 1;
+            const double run = prefix[lo] + (l0 ? __shfl(inc, l0 - 1, 64) : 0.0);
+            const uint64_t s = b + uint64_t(l0) * (kChunk / 64);
+            const uint64_t i = s + lane;
+            const double x = i < D ? p[i] : 0.0;
+            const double e = run + wave_incl_sum(x, lane);
+            hit = __ballot(i < D && e >= target);
+            if (hit) {  // (rounding may leave the last one below the target)
+                const int l = __ffsll(hit) - 1;
+                found = s + l;
+                e_at = __shfl(e, l, 64);
+                e_prev = __shfl(e - x, l, 64);
+            }
+        }
+        if (lane == 0) {
+            if (found == D) {
+                // past the end of the chunk: the sequential table's last entry is
+                // forced to 1, so the answer is certain only away from the edge
+                idx[shot] = D - 1;
+                certain[shot] = 0;
+            } else {
+                idx[shot] = found;
+                const double lo_edge = e_prev / total, hi_edge = e_at / total;
+                certain[shot] = (lo_edge < uu - B) && (hi_edge >= uu + B) &&
+                                (found != D - 1 || hi_edge >= uu + B);
+            }
         }
     }
 }
@@ -392,18 +394,19 @@ __global__ __launch_bounds__(kExN) void k_ex_chain(const double* __restrict__ p,
 __global__ __launch_bounds__(256) void k_ex_find(const double* __restrict__ s_in, uint64_t nb,
                                                  const double* __restrict__ u, uint64_t nshots,
                                                  uint32_t* __restrict__ blk) {
-    const uint64_t s = uint64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (s >= nshots) return;
-    const double us = u[s];
-    uint64_t lo = 0, hi = nb;  // s_in[lo] < us, or lo == 0
-    while (hi - lo > 1) {
-        const uint64_t mid = lo + (hi - lo) / 2;
-        if (s_in[mid] < us)
-            lo = mid;
-        else
-            hi = mid;
+    const uint64_t stride = uint64_t(gridDim.x) * 256;
+    for (uint64_t s = uint64_t(blockIdx.x) * 256 + threadIdx.x; s < nshots; s += stride) {
+        const double us = u[s];
+        uint64_t lo = 0, hi = nb;  // s_in[lo] < us, or lo == 0
+        while (hi - lo > 1) {
+            const uint64_t mid = lo + (hi - lo) / 2;
+            if (s_in[mid] < us)
+                lo = mid;
+            else
+                hi = mid;
+        }
+        blk[s] = static_cast<uint32_t>(lo);
     }
-    blk[s] = static_cast<uint32_t>(lo);
 }
 
 // One block's exact table in LDS (the table of all blocks in HBM, and a

@@ -63,3 +63,23 @@ def test_forced_exact_table_matches_oracle(qa, orc, mode, n, monkeypatch):
     monkeypatch.delenv("QPP_AMD_FORCE_EXACT")
     idx2, _, _ = st.sample(list(range(n)), u)
     assert np.array_equal(idx, idx2)
+
+
+@pytest.mark.parametrize("forced,n,nshots", [(False, 10, 262144), (False, 10, 300001), (True, 10, 300001),
+                                             (False, 3, 2 ** 24 + 777), (True, 3, 2 ** 24 + 777)])
+def test_more_shots_than_one_launch_of_waves(qa, orc, forced, n, nshots, monkeypatch):
+    """More shots than the searches' grids hold at one a wave (262144) or one
+    a thread (2^24): every shot is searched and equals the oracle's table."""
+    print(f"many shots: forced={forced} n={n} shots={nshots}", flush=True)
+    rng = np.random.default_rng(n)
+    # another call first, whose workspace the pool may hand out again
+    qa.State.from_array(randket(2 ** 9, rng), [2] * 9).sample([0], rng.random(1000))
+    if forced:
+        monkeypatch.setenv("QPP_AMD_FORCE_EXACT", "1")
+    psi = randket(2 ** n, rng)
+    p = orc.probs(psi)
+    u = rng.random(nshots)
+    idx, _, pr = qa.State.from_array(psi, [2] * n).sample([0], u)
+    ref = np.searchsorted(orc.discrete_table(p), u, side="left")
+    assert np.array_equal(idx, ref.astype(np.uint64))
+    assert np.array_equal(pr, p[ref])
