@@ -221,13 +221,17 @@ __global__ __launch_bounds__(256) void k_search(const double* __restrict__ p,
     }
 }
 
-// p[idx[s]] for every shot
-__global__ __launch_bounds__(256) void k_gather(const double* __restrict__ p,
+// p[idx[s]] for every shot, from the state (w.p may hold the exact table)
+template <typename T>
+__global__ __launch_bounds__(256) void k_gather(const T* __restrict__ a, uint64_t D, int rho,
                                                 const uint64_t* __restrict__ idx, uint64_t n,
                                                 double* __restrict__ out) {
     const uint64_t stride = uint64_t(gridDim.x) * 256;
-    for (uint64_t s = uint64_t(blockIdx.x) * 256 + threadIdx.x; s < n; s += stride)
-        out[s] = p[idx[s]];
+    for (uint64_t s = uint64_t(blockIdx.x) * 256 + threadIdx.x; s < n; s += stride) {
+        const uint64_t i = idx[s];
+        const T v = a[rho ? i + i * D : i];
+        out[s] = rho ? static_cast<double>(v.x) : norm_exact(v.x, v.y);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -245,7 +249,9 @@ __global__ __launch_bounds__(256) void k_gather(const double* __restrict__ p,
 //   k_ex_find      the block of every shot, by the blocks' exact entry values;
 //   k_ex_pick      rebuilds the cp of the blocks that have shots from their
 //                  entry values (wg_chunk), in LDS, and finds each shot's
-//                  lower_bound(cp, u) there.
+//                  lower_bound(cp, u) there;
+//   k_ex_expand, k_ex_search  instead of these two for many shots: the cp of
+//                  all blocks, in place of p, and a search of it.
 // The approximate prefix only picks the binade a block's map is built in;
 // a wrong pick sends the block to the element path and never changes a
 // result.  Element k of the summed sequence is p_k (S == nullptr) or
@@ -409,9 +415,9 @@ __global__ __launch_bounds__(256) void k_ex_find(const double* __restrict__ s_in
     }
 }
 
-// One block's exact table in LDS (the table of all blocks in HBM, and a
-// search of it, took 145 us at 2^24 elements, this 41-99), and in it the index of one shot (PERSHOT:
-// workgroup s takes shot s) or of all shots of the block (workgroup b).
+// Few shots: one block's exact table in LDS, and in it the index of one shot
+// (PERSHOT: workgroup s takes shot s) or of all shots of the block (workgroup
+// b, which looks through all shots for its own).
 template <bool PERSHOT>
 __global__ __launch_bounds__(256) void k_ex_pick(const double* __restrict__ p, uint64_t D,
                                                  const double* __restrict__ S,
@@ -461,6 +467,44 @@ __global__ __launch_bounds__(256) void k_ex_pick(const double* __restrict__ p, u
             idx[s] = i0 + (lo < n ? lo : n - 1);
         }
         __syncthreads();  // L and cp are used again
+    }
+}
+
+// Many shots: every block turns its p into the exact table, in place, and
+// k_ex_search finds every shot in it.
+__global__ __launch_bounds__(256) void k_ex_expand(double* p, uint64_t D, const double* __restrict__ S,
+                                                   const double* __restrict__ s_in, uint64_t nb) {
+    using namespace qs_exact;
+    __shared__ ChunkLds<256> L;
+    const double sv = *S;
+    for (uint64_t b = blockIdx.x; b < nb; b += gridDim.x) {
+        double x[kExV], out[kExV];
+        ex_load(p, D, S, sv, b, x);
+        (void)wg_chunk<256, kExV>(s_in[b], x, out, L);
+        const uint64_t i0 = b * kChunk + uint64_t(threadIdx.x) * kExV;
+#pragma unroll
+        for (int j = 0; j < kExV; ++j)
+            if (i0 + j < D) p[i0 + j] = i0 + j == D - 1 ? 1.0 : out[j];
+        __syncthreads();  // L is used again
+    }
+}
+
+// first k with cp[k] >= u[s] (cp[D-1] == 1 > u)
+__global__ __launch_bounds__(256) void k_ex_search(const double* __restrict__ cp, uint64_t D,
+                                                   const double* __restrict__ u, uint64_t nshots,
+                                                   uint64_t* __restrict__ idx) {
+    const uint64_t stride = uint64_t(gridDim.x) * 256;
+    for (uint64_t s = uint64_t(blockIdx.x) * 256 + threadIdx.x; s < nshots; s += stride) {
+        const double us = u[s];
+        uint64_t lo = 0, hi = D;
+        while (lo < hi) {
+            const uint64_t mid = lo + (hi - lo) / 2;
+            if (cp[mid] < us)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        idx[s] = lo < D ? lo : D - 1;
     }
 }
 
@@ -779,7 +823,7 @@ double bound_for(uint64_t N) {
 // Device workspace of one sample_device call, carved from one allocation
 // (256-byte aligned segments).
 struct SampleWs {
-    double* p;       // D probabilities
+    double* p;       // D probabilities, then (k_ex_expand) the exact table
     double* sums;    // nchunks block sums
     double* prefix;  // nchunks + 1: their exclusive prefix and total
     qs_exact::Tr* T; // nchunks block maps
@@ -788,7 +832,7 @@ struct SampleWs {
     double* sq_in;   // nchunks + 1: the same for p / S
     double* u;       // nshots uniforms (then the gathered probabilities)
     uint64_t* idx;   // nshots indices
-    int* cert;       // nshots: decided by the approximate search, then the shot's block
+    int* cert;       // nshots: decided by the approximate search, then (k_ex_find) the shot's block
 };
 
 constexpr size_t align256(size_t v) { return (v + 255) / 256 * 256; }
@@ -847,8 +891,29 @@ int probs_sums(const qs_state* st, const SampleWs& w, uint64_t nchunks) {
     return QS_OK;
 }
 
+// Probabilities of the shots' indices, over their uniforms.
+int gather_probs(const qs_state* st, const SampleWs& w, uint64_t nshots) {
+    const dim3 g(grid_for(nshots, 256));
+    const int rho = st->kind == QS_RHO;
+    if (st->dtype == QS_C128)
+        hipLaunchKernelGGL(k_gather<double2>, g, dim3(256), 0, st->stream, static_cast<const double2*>(st->d),
+                           st->D, rho, w.idx, nshots, w.u);
+    else
+        hipLaunchKernelGGL(k_gather<float2>, g, dim3(256), 0, st->stream, static_cast<const float2*>(st->d),
+                           st->D, rho, w.idx, nshots, w.u);
+    QS_HIP(hipGetLastError(), "qpp::sample()");
+    return QS_OK;
+}
+
 // Every shot's index in the exact table (k_ex_* above).  Needs w.p, w.prefix
-// (k_probs_sums + k_scan_chunks) and w.u.
+// (k_probs_sums + k_scan_chunks) and w.u; w.p may hold the table afterwards.
+// Rebuilding the blocks that have shots costs more with every shot, the table
+// of all blocks by their number.  us of k_ex_find and k_ex_pick against
+// k_ex_expand and k_ex_search, 22 qubits: 90 and 123 (1024 shots), 122 and
+// 123 (4096), 131 and 124 (8192); 24 qubits: 84 and 148, 118 and 150, 163 and
+// 149; 262144 shots of 8, 14, 20 and 24 qubits: 1300 and 34, 1640 and 107,
+// 1415 and 105, 3250 and 161.
+constexpr uint64_t kExFewShots = 4096;
 int exact_table_search(const qs_state* st, const SampleWs& w, uint64_t nshots) {
     const uint64_t D = st->D;
     const uint64_t nb = (D + kChunk - 1) / kChunk;
@@ -862,15 +927,20 @@ int exact_table_search(const qs_state* st, const SampleWs& w, uint64_t nshots) {
     hipLaunchKernelGGL(k_ex_block_tr, dim3(g), dim3(256), 0, sm, w.p, D, S, w.prefix, nb, w.T,
                        w.Eb);
     hipLaunchKernelGGL(k_ex_chain, dim3(1), dim3(kExN), 0, sm, w.p, D, S, nb, w.T, w.Eb, w.sq_in);
-    auto* blk = reinterpret_cast<uint32_t*>(w.cert);
-    hipLaunchKernelGGL(k_ex_find, dim3(grid_for(nshots, 256)), dim3(256), 0, sm, w.sq_in, nb, w.u, nshots, blk);
-    // a workgroup per shot or per block, whichever are fewer
-    if (nshots < nb)
-        hipLaunchKernelGGL(k_ex_pick<true>, dim3(grid_for(nshots, 1)), dim3(256), 0, sm, w.p, D, S, w.sq_in, nb,
-                           w.u, nshots, blk, w.idx);
-    else
-        hipLaunchKernelGGL(k_ex_pick<false>, dim3(g), dim3(256), 0, sm, w.p, D, S, w.sq_in, nb, w.u, nshots, blk,
-                           w.idx);
+    if (nshots > kExFewShots + 3 * nb / 4) {
+        hipLaunchKernelGGL(k_ex_expand, dim3(g), dim3(256), 0, sm, w.p, D, S, w.sq_in, nb);
+        hipLaunchKernelGGL(k_ex_search, dim3(grid_for(nshots, 256)), dim3(256), 0, sm, w.p, D, w.u, nshots, w.idx);
+    } else {
+        auto* blk = reinterpret_cast<uint32_t*>(w.cert);
+        hipLaunchKernelGGL(k_ex_find, dim3(grid_for(nshots, 256)), dim3(256), 0, sm, w.sq_in, nb, w.u, nshots, blk);
+        // a workgroup per shot or per block, whichever are fewer
+        if (nshots < nb)
+            hipLaunchKernelGGL(k_ex_pick<true>, dim3(grid_for(nshots, 1)), dim3(256), 0, sm, w.p, D, S, w.sq_in, nb,
+                               w.u, nshots, blk, w.idx);
+        else
+            hipLaunchKernelGGL(k_ex_pick<false>, dim3(g), dim3(256), 0, sm, w.p, D, S, w.sq_in, nb, w.u, nshots,
+                               blk, w.idx);
+    }
     QS_HIP(hipGetLastError(), "qpp::sample()");
     return QS_OK;
 }
@@ -927,9 +997,7 @@ int sample_device(const qs_state* st, const double* u_host, uint64_t nshots,
         // p[index] of every shot (instruments.hpp:808), gathered on the
         // device; the u slots are free once the searches have run
         if (out_prob_host) {
-            hipLaunchKernelGGL(k_gather, dim3(grid_for(nshots, 256)), dim3(256), 0, st->stream,
-                               w.p, w.idx, nshots, w.u);
-            QS_HIP(hipGetLastError(), "qpp::sample()");
+            if (int rc = gather_probs(st, w, nshots)) return rc;
             QS_HIP(hipMemcpyAsync(out_prob_host, w.u, nshots * 8, hipMemcpyDeviceToHost,
                                   st->stream),
                    "qpp::sample()");
@@ -1019,9 +1087,7 @@ int sample_exact_only(const qs_state* st, const double* u_host, uint64_t nshots,
     if (idx_host)
         QS_HIP(hipMemcpyAsync(idx_host, w.idx, nshots * 8, hipMemcpyDeviceToHost, st->stream), W);
     if (prob_host) {
-        hipLaunchKernelGGL(k_gather, dim3(grid_for(nshots, 256)), dim3(256), 0, st->stream, w.p,
-                           w.idx, nshots, w.u);
-        QS_HIP(hipGetLastError(), W);
+        if (int rc = gather_probs(st, w, nshots)) return rc;
         QS_HIP(hipMemcpyAsync(prob_host, w.u, nshots * 8, hipMemcpyDeviceToHost, st->stream), W);
     }
     QS_HIP(hipStreamSynchronize(st->stream), W);

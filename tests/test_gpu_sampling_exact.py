@@ -83,3 +83,28 @@ def test_more_shots_than_one_launch_of_waves(qa, orc, forced, n, nshots, monkeyp
     ref = np.searchsorted(orc.discrete_table(p), u, side="left")
     assert np.array_equal(idx, ref.astype(np.uint64))
     assert np.array_equal(pr, p[ref])
+
+
+@pytest.mark.parametrize("kind,n,nshots", [
+    ("ket", 3, 4096), ("ket", 3, 4097), ("ket", 12, 4096), ("ket", 12, 4097), ("ket", 12, 20000), ("ket", 13, 4098),
+    ("ket", 14, 4099), ("ket", 14, 4100), ("ket", 20, 4288), ("ket", 20, 4289), ("ket", 20, 255), ("ket", 20, 256),
+    ("c64", 13, 3000), ("c64", 13, 9000), ("rho", 5, 4097), ("rho", 7, 100), ("rho", 7, 6000)])
+def test_exact_table_by_number_of_shots(qa, orc, kind, n, nshots, monkeypatch):
+    """The exact table's three ways (a workgroup per shot, per block, the
+    whole table) at the shot counts where one takes over from another: equal
+    to the oracle's table, with the probabilities of the state."""
+    monkeypatch.setenv("QPP_AMD_FORCE_EXACT", "1")
+    rng = np.random.default_rng(n + nshots)
+    psi = randket(2 ** n, rng)
+    if kind == "c64":
+        psi = psi.astype(np.complex64).astype(np.complex128)
+    A = np.outer(psi, psi.conj()) if kind == "rho" else psi
+    p = orc.probs(A)
+    u = np.concatenate([[0.0, np.nextafter(1.0, 0)], rng.random(nshots - 2)])
+    st = qa.State.from_array(A, [2] * n, dtype=qa.C64 if kind == "c64" else qa.C128)
+    print(f"exact table: {kind} n={n} shots={nshots}", flush=True)
+    for _ in range(2):  # the state is unchanged by a call
+        idx, _, pr = st.sample([0], u)
+        ref = np.searchsorted(orc.discrete_table(p), u, side="left")
+        assert np.array_equal(idx, ref.astype(np.uint64))
+        assert np.array_equal(pr, p[ref])
