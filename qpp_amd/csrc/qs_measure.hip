@@ -152,8 +152,15 @@ __global__ __launch_bounds__(1024) void k_scan_chunks(const double* __restrict__
 }
 
 // One wave per shot (a grid of waves over all shots): binary search over
-// chunk prefixes, then an in-chunk wave scan.  Writes the candidate index and
-// whether it is certain.
+// chunk prefixes, then the first E_k >= target within the chunk.  Writes the
+// candidate index and whether it is certain.  MANY: the chunk is scanned 64
+// consecutive elements at a time until the target is met, coalesced loads
+// that depend on each other.  Else the lanes load and sum 64 elements each,
+// all loads in flight at once but a line to a lane, and one group of 64 is
+// scanned.  us with many and with few waves: 1024 shots 42 and 14 (20
+// qubits), 12 and 8 (10); 4096 48 and 43, 13 and 18; 8192 70 and 77, 16 and
+// 30; 262144 1384 and 2108, 216 and 835.
+template <bool MANY>
 __global__ __launch_bounds__(256) void k_search(const double* __restrict__ p,
                                                 uint64_t D,
                                                 const double* __restrict__ prefix,
@@ -177,32 +184,51 @@ __global__ __launch_bounds__(256) void k_search(const double* __restrict__ p,
             else
                 hi = mid;
         }
-        // the 64 elements of the chunk that hold the first E_k >= target: each
-        // lane sums 64 consecutive ones; then those, one a lane
         const uint64_t b = lo * kChunk;
-        double v = 0;
-#pragma unroll 16
-        for (int j = 0; j < kChunk / 64; ++j) {
-            const uint64_t i = b + uint64_t(lane) * (kChunk / 64) + j;
-            v += i < D ? p[i] : 0.0;
-        }
-        const double inc = wave_incl_sum(v, lane);
-        unsigned long long hit = __ballot(prefix[lo] + inc >= target);
         uint64_t found = D;  // D = not found in this chunk
         double e_prev = 0, e_at = 0;
-        if (hit) {
-            const int l0 = __ffsll(hit) - 1;
-            const double run = prefix[lo] + (l0 ? __shfl(inc, l0 - 1, 64) : 0.0);
-            const uint64_t s = b + uint64_t(l0) * (kChunk / 64);
-            const uint64_t i = s + lane;
-            const double x = i < D ? p[i] : 0.0;
-            const double e = run + wave_incl_sum(x, lane);
-            hit = __ballot(i < D && e >= target);
-            if (hit) {  // (rounding may leave the last one below the target)
-                const int l = __ffsll(hit) - 1;
-                found = s + l;
-                e_at = __shfl(e, l, 64);
-                e_prev = __shfl(e - x, l, 64);
+        if constexpr (MANY) {
+            double run = prefix[lo];
+            for (uint64_t s = b; s < b + kChunk && s < D; s += 64) {
+                const uint64_t i = s + lane;
+                const double x = i < D ? p[i] : 0.0;
+                const double inc = wave_incl_sum(x, lane);
+                const double e = run + inc;
+                const unsigned long long hit = __ballot(i < D && e >= target);
+                if (hit) {
+                    const int l = __ffsll(hit) - 1;
+                    found = s + l;
+                    e_at = __shfl(e, l, 64);
+                    e_prev = __shfl(e - x, l, 64);
+                    break;
+                }
+                run += __shfl(inc, 63, 64);
+            }
+        } else {
+            // the 64 elements of the chunk that hold the first E_k >= target: each
+            // lane sums 64 consecutive ones; then those, one a lane
+            double v = 0;
+#pragma unroll 16
+            for (int j = 0; j < kChunk / 64; ++j) {
+                const uint64_t i = b + uint64_t(lane) * (kChunk / 64) + j;
+                v += i < D ? p[i] : 0.0;
+            }
+            const double inc = wave_incl_sum(v, lane);
+            unsigned long long hit = __ballot(prefix[lo] + inc >= target);
+            if (hit) {
+                const int l0 = __ffsll(hit) - 1;
+                const double run = prefix[lo] + (l0 ? __shfl(inc, l0 - 1, 64) : 0.0);
+                const uint64_t s = b + uint64_t(l0) * (kChunk / 64);
+                const uint64_t i = s + lane;
+                const double x = i < D ? p[i] : 0.0;
+                const double e = run + wave_incl_sum(x, lane);
+                hit = __ballot(i < D && e >= target);
+                if (hit) {  // (rounding may leave the last one below the target)
+                    const int l = __ffsll(hit) - 1;
+                    found = s + l;
+                    e_at = __shfl(e, l, 64);
+                    e_prev = __shfl(e - x, l, 64);
+                }
             }
         }
         if (lane == 0) {
@@ -978,8 +1004,9 @@ int sample_device(const qs_state* st, const double* u_host, uint64_t nshots,
         hipLaunchKernelGGL(k_scan_chunks, dim3(1), dim3(1024), 0, st->stream, w.sums, nchunks,
                            w.prefix);
         const double B = bound_for(D);
-        hipLaunchKernelGGL(k_search, dim3(grid_for(nshots * 64, 256)), dim3(256), 0, st->stream,
-                           w.p, D, w.prefix, nchunks, w.u, nshots, B, w.idx, w.cert);
+        const bool many = nshots > 4096 || (nshots > 1024 && D <= 1024);  // (see k_search)
+        hipLaunchKernelGGL(many ? k_search<true> : k_search<false>, dim3(grid_for(nshots * 64, 256)), dim3(256), 0,
+                           st->stream, w.p, D, w.prefix, nchunks, w.u, nshots, B, w.idx, w.cert);
         QS_HIP(hipGetLastError(), "qpp::sample()");
         std::vector<int> hc(nshots);
         QS_HIP(hipMemcpyAsync(hc.data(), w.cert, nshots * 4, hipMemcpyDeviceToHost, st->stream),

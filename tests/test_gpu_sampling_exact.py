@@ -108,3 +108,18 @@ def test_exact_table_by_number_of_shots(qa, orc, kind, n, nshots, monkeypatch):
         ref = np.searchsorted(orc.discrete_table(p), u, side="left")
         assert np.array_equal(idx, ref.astype(np.uint64))
         assert np.array_equal(pr, p[ref])
+
+
+@pytest.mark.parametrize("n,nshots", [(2, 1025), (10, 1024), (10, 1025), (11, 1025), (13, 4096), (13, 4097),
+                                      (17, 5000)])
+def test_search_by_number_of_shots(qa, orc, n, nshots):
+    """The error-bounded search's two ways through a chunk, at the shot
+    counts where one takes over: indices equal the oracle's table."""
+    rng = np.random.default_rng(n + nshots)
+    psi = make_state("random", n, rng)
+    p = orc.probs(psi)
+    u = rng.random(nshots)
+    print(f"search: n={n} shots={nshots}", flush=True)
+    idx, _, pr = qa.State.from_array(psi, [2] * n).sample([0], u)
+    ref = np.searchsorted(orc.discrete_table(p), u, side="left")
+    assert np.array_equal(idx, ref.astype(np.uint64)) and np.array_equal(pr, p[ref])
