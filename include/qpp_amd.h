@@ -479,7 +479,7 @@ int qs_engine_set_limits(qs_engine* e, uint64_t max_loop_reps, uint64_t max_ps_f
 int qs_engine_noise_results(const qs_engine* e, uint64_t step, uint64_t* out, uint64_t* count);
 
 /* ------------------------------------------------------------------------ */
-/* Batched noisy trajectories (one persistent launch)                        */
+/* Batched noisy trajectories                                                */
 /* ------------------------------------------------------------------------ */
 /* Trajectory i of a run computes what
  *   QNoisyEngine<QubitDepolarizingNoise(noise_p)>(circuits[circuit_of[i]],
@@ -491,6 +491,10 @@ int qs_engine_noise_results(const qs_engine* e, uint64_t step, uint64_t* out, ui
  * steps whose gates are dense 1-qubit gates or Clifford gates on at most 2
  * qubits (CNOT, CZ, X, Z, ...), ending in one MEASURE_MANY of every qubit.
  * Circuits may have different qubit counts (>= 8 + reg_bits).
+ * One persistent launch runs the trajectories, a workgroup each; those of 18
+ * qubits and more, and smaller ones where that is faster, run pass by pass on
+ * device states of their own first (the smaller ones in runs of at most 1 GiB
+ * of states, or what the launch itself would hold for them).
  * out_index[i]: basis index of the outcome (measured digit of target j =
  * bit (n-1-target[j])); out_prob[i]: its probability. */
 typedef struct qs_batch qs_batch;

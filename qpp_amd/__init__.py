@@ -1209,7 +1209,7 @@ class QEngine:
 
 
 class Batch:
-    """Batched noisy trajectories in one persistent launch.  Trajectory i is
+    """Batched noisy trajectories in one call.  Trajectory i is
     QNoisyEngine<QubitDepolarizingNoise(noise_p)>(circuits[circuit_of[i]],
     seed=seeds[i]).execute(1) (noise_p < 0: QEngine(...).execute(1));
     every circuit ends in one measurement of all its qubits."""

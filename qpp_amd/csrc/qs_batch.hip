@@ -675,6 +675,7 @@ struct qs_batch {
     size_t c_wend = 0;
     // class -> offsets of its passes and ops in the concatenated tables
     std::vector<int> pass_base, op_base;
+    int ncu = 0, traj_per_cu = 0;  // the device's CUs, k_traj's workgroups on one (launch_limits)
     // last run
     uint64_t last_exact = 0;
     double last_host_ms = 0, last_device_ms = 0;
@@ -949,13 +950,70 @@ bool small_go_wide(const qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of
     return wide <= std::max(longest, all / double(2 * ncu));
 }
 
+// b->ncu and b->traj_per_cu
+int launch_limits(qs_batch* b) {
+    constexpr const char* W = "qpp_amd::batch";
+    if (b->ncu) return QS_OK;
+    if (int rc = qs::ensure_device()) return rc;
+    const size_t shmem = (b->dtype == QS_C128 ? size_t{16} : size_t{8}) << (8 + b->reg_bits);
+    int dev = 0, ncu = 0, per_cu = 0;
+    QS_HIP(hipGetDevice(&dev), W);
+    QS_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), W);
+    hipError_t e;
+    if (b->dtype == QS_C128)
+        e = b->reg_bits == 3
+                ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<double, 8>, kThreads, shmem)
+                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<double, 16>, kThreads, shmem);
+    else
+        e = b->reg_bits == 3
+                ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<float, 8>, kThreads, shmem)
+                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<float, 16>, kThreads, shmem);
+    if (e != hipSuccess) return qs::fail_hip(e, W);
+    b->traj_per_cu = std::max(1, per_cu);
+    b->ncu = std::max(1, ncu);
+    return QS_OK;
+}
+
+// Workgroups of k_traj for ntraj trajectories.
+uint64_t traj_grid(const qs_batch* b, uint64_t ntraj) {
+    return std::max<uint64_t>(1, std::min<uint64_t>(ntraj, uint64_t(b->traj_per_cu) * uint64_t(b->ncu)));
+}
+
+// The qubit count from which trajectories run pass by pass.
+uint32_t wide_from(const qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of) {
+    uint32_t bits = 0;
+    if (wide_bits_set(&bits)) return bits;
+    return small_go_wide(b, ntraj, circuit_of, uint64_t(b->ncu)) ? 0 : kWideBits;
+}
+
+// Bytes of states that small trajectories may hold at a time when they run
+// pass by pass: what their slots in the persistent launch would take, or 1
+// GiB (runs of few states leave the chip idle at their ends: 10000
+// trajectories of 12 qubits in runs of the slots' size 12.5 ms, in one run
+// 8.0, persistent 9.1, complex64).  The environment variable
+// QPP_AMD_TRAJ_STATES_BYTES sets another amount (0: none of their own).
+uint64_t small_room(uint64_t slots) {
+    const char* v = std::getenv("QPP_AMD_TRAJ_STATES_BYTES");
+    if (v && *v) return std::strtoull(v, nullptr, 10);
+    return std::max(slots, uint64_t{1} << 30);
+}
+
+// run_impl: no memory for the small trajectories' states
+constexpr int kNoRoom = -1;
+
+void give_back(void*& d, size_t& cap, hipStream_t s) {
+    if (d) (void)hipFreeAsync(d, s);
+    d = nullptr;
+    cap = 0;
+}
+
 // One launch of k_traj over ntraj trajectories (arguments validated by the
-// caller), after the passes of the wide ones.  dst: nullptr (each
-// trajectory ends in its measurement), or one state per trajectory that
-// receives its final state instead (the wide ones' passes then run on it
-// and k_traj leaves them alone).
-int run_impl(qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, const uint64_t* seeds,
-             double noise_p, const std::vector<void*>* dst, uint64_t* out_index, double* out_prob) {
+// caller), after the passes of the wide ones (of at least wbits qubits).
+// dst: nullptr (each trajectory ends in its measurement), or one state per
+// trajectory that receives its final state instead (the wide ones' passes
+// then run on it and k_traj leaves them alone).
+int run_impl(qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, const uint64_t* seeds, double noise_p,
+             uint32_t wbits, const std::vector<void*>* dst, uint64_t* out_index, double* out_prob) {
     constexpr const char* W = "qpp_amd::batch";
     if (int rc = qs::ensure_device()) return rc;
     if (!b->stream) b->stream = qs::current_stream();
@@ -996,12 +1054,6 @@ int run_impl(qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, const uint
     std::vector<uint32_t> order(ntraj);
     std::iota(order.begin(), order.end(), 0u);
     // wide trajectories, grouped by circuit: their passes run before k_traj
-    int dev = 0, ncu = 0;
-    QS_HIP(hipGetDevice(&dev), W);
-    QS_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), W);
-    uint32_t wbits = 0;
-    if (!wide_bits_set(&wbits))
-        wbits = small_go_wide(b, ntraj, circuit_of, std::max(1, ncu)) ? 0 : kWideBits;
     std::vector<uint32_t> wide;
     std::vector<char> is_wide(ntraj, 0);
     for (uint64_t i = 0; i < ntraj; ++i) {
@@ -1027,24 +1079,14 @@ int run_impl(qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, const uint
         if (!is_wide[i]) maxnb = std::max(maxnb, b->cls[circuit_of[i]].nb);
     const size_t es = b->dtype == QS_C128 ? 16 : 8;
     const size_t shmem = es << (8 + b->reg_bits);
-    int per_cu = 0;
-    hipError_t e;
-    if (b->dtype == QS_C128)
-        e = b->reg_bits == 3
-                ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<double, 8>, kThreads, shmem)
-                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<double, 16>, kThreads, shmem);
-    else
-        e = b->reg_bits == 3
-                ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<float, 8>, kThreads, shmem)
-                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<float, 16>, kThreads, shmem);
-    if (e != hipSuccess) return qs::fail_hip(e, W);
-    const uint64_t grid = std::max<uint64_t>(1, std::min<uint64_t>(ntraj, uint64_t(std::max(1, per_cu)) * ncu));
+    const uint64_t grid = traj_grid(b, ntraj);
     const uint64_t slot = uint64_t{1} << maxnb;
     const size_t ws_bytes = dst ? 0 : size_t(grid) * slot * es;
+    // what an earlier run of the other kind held is given back first
+    if (wide.size() == ntraj) give_back(b->d_ws, b->c_ws, s);
+    if (wide.empty()) give_back(b->d_wide, b->c_wide, s);
     if (ws_bytes > b->c_ws) {
-        if (b->d_ws) (void)hipFreeAsync(b->d_ws, s);
-        b->d_ws = nullptr;
-        b->c_ws = 0;
+        give_back(b->d_ws, b->c_ws, s);
         QS_HIP(hipMallocAsync(&b->d_ws, ws_bytes, s), W);
         b->c_ws = ws_bytes;
     }
@@ -1061,10 +1103,14 @@ int run_impl(qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, const uint
         if (!dst)
             for (uint32_t i : wide) wbytes += es << b->cls[circuit_of[i]].nb;
         if (wbytes > b->c_wide) {
-            if (b->d_wide) (void)hipFreeAsync(b->d_wide, s);
-            b->d_wide = nullptr;
-            b->c_wide = 0;
-            QS_HIP(hipMallocAsync(&b->d_wide, wbytes, s), W);
+            give_back(b->d_wide, b->c_wide, s);
+            const hipError_t e = hipMallocAsync(&b->d_wide, wbytes, s);
+            if (e != hipSuccess) {
+                b->d_wide = nullptr;
+                if (wbits != 0 || e != hipErrorOutOfMemory) return qs::fail_hip(e, W);
+                (void)hipGetLastError();  // handled: not the next call's
+                return kNoRoom;
+            }
             b->c_wide = wbytes;
         }
         src.assign(ntraj, nullptr);
@@ -1190,7 +1236,7 @@ int run_impl(qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, const uint
                                static_cast<float2* const*>(dst ? b->d_dst : nullptr),
                                static_cast<float2* const*>(wide.empty() ? nullptr : b->d_src));
     }
-    e = hipGetLastError();
+    hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipEventRecord(e1, s);
     std::vector<TrajOut> res(ntraj);
     if (e == hipSuccess) e = hipMemcpyAsync(res.data(), outp, ob, hipMemcpyDeviceToHost, s);
@@ -1226,31 +1272,71 @@ int qs_batch_run(qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, const 
     if (!(noise_p <= 1.0)) return fail(QS_ERR_OUT_OF_RANGE, W, "noise_p");
     for (uint64_t i = 0; i < ntraj; ++i)
         if (circuit_of[i] >= b->cls.size()) return fail(QS_ERR_OUT_OF_RANGE, W, "circuit_of");
-    // Pass by pass, every trajectory has a state of its own: those of fewer
-    // than kWideBits qubits are taken in runs of at most 4 GiB of states
-    // (some thousand trajectories at least).
-    constexpr uint64_t kMost = uint64_t{4} << 30;
+    if (int rc = launch_limits(b)) return rc;
+    const uint32_t wbits = wide_from(b, ntraj, circuit_of);
+    if (wbits != 0)
+        return run_impl(b, ntraj, circuit_of, seeds, noise_p, wbits, nullptr, out_index, out_prob);
+    // Pass by pass, every trajectory has a state of its own.  Those of fewer
+    // than kWideBits qubits are taken in runs of at most small_room bytes of
+    // states; the wider ones, which hold their states in any case, go with
+    // the first run.  Where a run finds no memory, what is left goes into the
+    // persistent launch on its slots.
+    const size_t es = b->dtype == QS_C128 ? 16 : 8;
+    std::vector<uint64_t> take, small;
+    uint32_t maxnb = 0;
+    for (uint64_t i = 0; i < ntraj; ++i) {
+        const uint32_t nb = b->cls[circuit_of[i]].nb;
+        (nb < kWideBits ? small : take).push_back(i);
+        if (nb < kWideBits) maxnb = std::max(maxnb, nb);
+    }
+    const uint64_t slots = traj_grid(b, ntraj) * es << maxnb, room = small_room(slots);
     uint64_t exact = 0;
     double host = 0, device = 0;
-    for (uint64_t i0 = 0, i1; i0 < ntraj; i0 = i1) {
-        uint64_t bytes = 0;
-        for (i1 = i0; i1 < ntraj; ++i1) {
-            const uint32_t nb = b->cls[circuit_of[i1]].nb;
-            const uint64_t need = nb < kWideBits ? (b->dtype == QS_C128 ? 16u : 8u) * (uint64_t{1} << nb) : 0;
-            if (bytes + need > kMost) break;
-            bytes += need;
+    auto run = [&](uint32_t from) {
+        const size_t n = take.size();
+        std::vector<uint32_t> cof(n);
+        std::vector<uint64_t> sd(n), index(n);
+        std::vector<double> prob(n);
+        for (size_t k = 0; k < n; ++k) {
+            cof[k] = circuit_of[take[k]];
+            sd[k] = seeds[take[k]];
         }
-        if (int rc = run_impl(b, i1 - i0, circuit_of + i0, seeds + i0, noise_p, nullptr,
-                              out_index ? out_index + i0 : nullptr, out_prob ? out_prob + i0 : nullptr))
+        if (int rc = run_impl(b, n, cof.data(), sd.data(), noise_p, from, nullptr, index.data(), prob.data()))
             return rc;
+        for (size_t k = 0; k < n; ++k) {
+            if (out_index) out_index[take[k]] = index[k];
+            if (out_prob) out_prob[take[k]] = prob[k];
+        }
+        take.clear();
         exact += b->last_exact;
         host += b->last_host_ms;
         device += b->last_device_ms;
+        return int(QS_OK);
+    };
+    size_t at = 0;
+    int rc = QS_OK;
+    while (rc == QS_OK && at < small.size()) {
+        const size_t first = at, wide = take.size();
+        for (uint64_t bytes = 0; at < small.size(); ++at) {
+            bytes += es << b->cls[circuit_of[small[at]]].nb;
+            if (bytes > room) break;
+            take.push_back(small[at]);
+        }
+        rc = at > first ? run(0) : kNoRoom;
+        if (rc == kNoRoom) {
+            take.resize(wide);
+            take.insert(take.end(), small.begin() + static_cast<std::ptrdiff_t>(first), small.end());
+            at = small.size();
+            rc = run(kWideBits);
+        }
     }
+    if (rc == QS_OK && !take.empty()) rc = run(kWideBits);  // (wide ones only)
+    // the pool keeps the memory at hand for the next call
+    if (b->c_wide > slots) give_back(b->d_wide, b->c_wide, b->stream);
     b->last_exact = exact;
     b->last_host_ms = host;
     b->last_device_ms = device;
-    return QS_OK;
+    return rc;
 }
 
 // The gate steps of circuit circuit_of[i] applied to |0..0> into out[i] (a
@@ -1280,8 +1366,10 @@ int qs_batch_run_states(qs_batch* b, uint64_t nstates, const uint32_t* circuit_o
     if (!b->stream) b->stream = qs::current_stream();
     for (uint64_t i = 0; i < nstates; ++i)
         if (out[i]->stream != b->stream) QS_HIP(hipStreamSynchronize(out[i]->stream), W);
+    if (int rc = launch_limits(b)) return rc;
     std::vector<uint64_t> seeds(nstates, 0);
-    return run_impl(b, nstates, circuit_of, seeds.data(), -1.0, &dst, nullptr, nullptr);
+    return run_impl(b, nstates, circuit_of, seeds.data(), -1.0, wide_from(b, nstates, circuit_of), &dst, nullptr,
+                    nullptr);
 }
 
 }  // extern "C"

@@ -7,6 +7,8 @@ from the same std::mt19937 stream (oracle Rng).  GPU: every trajectory's
 outcome equals the oracle QNoisyEngine's for the same seed, in the
 persistent launch and on the wide path (QPP_AMD_TRAJ_WIDE_BITS sets the
 qubit count from which trajectories run pass by pass; default 18)."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -201,13 +203,66 @@ def test_wide_trajectories_more_than_one_launch_row(monkeypatch):
 @pytest.mark.parametrize("n,ntr,depth", [(12, 1, 3), (13, 300, 2), (16, 40, 2), (17, 2100, 1)])
 def test_small_trajectories_by_rule(monkeypatch, n, ntr, depth):
     """Which way trajectories below the wide threshold run is chosen by
-    their number and tiles, and more than 4 GiB of their states are taken in
-    several runs; outcomes equal the persistent launch's bit for bit."""
+    their number and tiles, and many of their states are taken in several
+    runs; outcomes equal the persistent launch's bit for bit."""
     b = qa.Batch([noisy_circuit(n, depth, seed=91), noisy_circuit(12, 2, seed=92)], dtype=qa.C128)
     cof = np.array([int(i % 7 == 3) for i in range(ntr)], dtype=np.uint32)
     seeds = np.arange(ntr, dtype=np.uint64) + 99
     i0, p0 = b.run(cof, seeds, 0.01)
     monkeypatch.setenv("QPP_AMD_TRAJ_WIDE_BITS", "64")
+    i1, p1 = b.run(cof, seeds, 0.01)
+    assert np.array_equal(i0, i1) and np.array_equal(p0, p1)
+
+
+@gpu
+def test_small_trajectories_bounded_memory(monkeypatch):
+    """Small trajectories run pass by pass hold at most 1 GiB of states at a
+    time (or what their slots in the persistent launch would take), and give
+    back what is more than these slots: the stream-ordered pool's high-water
+    mark and use, for 6000 trajectories of 14 qubits (1.5 GiB of states)."""
+    L, pool = qa.lib(), ctypes.c_void_p()
+    used_now, used_high = 7, 8  # hipMemPoolAttrUsedMemCurrent, UsedMemHigh
+
+    def used(attr):
+        v = ctypes.c_uint64(0)
+        assert L.hipMemPoolGetAttribute(pool, attr, ctypes.byref(v)) == 0
+        return v.value
+
+    def memory(b):
+        qa.synchronize()
+        zero = ctypes.c_uint64(0)
+        assert L.hipDeviceGetDefaultMemPool(ctypes.byref(pool), 0) == 0
+        assert L.hipMemPoolSetAttribute(pool, used_high, ctypes.byref(zero)) == 0
+        before = used(used_now)
+        out = b.run(cof, seeds, 0.01)
+        qa.synchronize()
+        return out, used(used_high) - before, used(used_now) - before
+
+    n, ntr = 14, 6000
+    qc = noisy_circuit(n, 2, seed=93)
+    cof, seeds = np.zeros(ntr, dtype=np.uint32), np.arange(ntr, dtype=np.uint64) + 5
+    monkeypatch.setenv("QPP_AMD_TRAJ_WIDE_BITS", "64")
+    (i0, p0), single, kept0 = memory(qa.Batch(qc, dtype=qa.C128))
+    monkeypatch.delenv("QPP_AMD_TRAJ_WIDE_BITS")
+    (i1, p1), high, kept1 = memory(qa.Batch(qc, dtype=qa.C128))
+    print(f"batch memory: persistent launch {single} B (kept {kept0}), by rule {high} B (kept {kept1})", flush=True)
+    assert np.array_equal(i0, i1) and np.array_equal(p0, p1)
+    more = 4 << 20  # tables and per-trajectory records
+    assert single >= 2 ** n * 16 and high <= max(single, 1 << 30) + more and kept1 <= kept0 + more
+
+
+@gpu
+@pytest.mark.parametrize("room", [0, 2 ** 13 * 16, 5 << 20])
+def test_small_trajectories_without_room(monkeypatch, room):
+    """Small trajectories whose states find no memory run in the persistent
+    launch, also beside wide ones; less room means more runs.  Outcomes are
+    the same."""
+    circs = [noisy_circuit(n, 2, seed=95 + n) for n in (12, 13, 14, 18)]
+    b = qa.Batch(circs, dtype=qa.C128)
+    cof = np.array([3 if i == 2 else i % 3 for i in range(60)], dtype=np.uint32)
+    seeds = np.arange(60, dtype=np.uint64) + 7
+    i0, p0 = b.run(cof, seeds, 0.01)
+    monkeypatch.setenv("QPP_AMD_TRAJ_STATES_BYTES", str(room))
     i1, p1 = b.run(cof, seeds, 0.01)
     assert np.array_equal(i0, i1) and np.array_equal(p0, p1)
 
