@@ -40,6 +40,7 @@
 #include <thread>
 #include <vector>
 
+#include "qs_batch_rule.hpp"
 #include "qs_fused.hpp"
 #include "qs_internal.hpp"
 #include "qs_exact.hpp"
@@ -675,7 +676,7 @@ struct qs_batch {
     size_t c_wend = 0;
     // class -> offsets of its passes and ops in the concatenated tables
     std::vector<int> pass_base, op_base;
-    int ncu = 0, traj_per_cu = 0;  // the device's CUs, k_traj's workgroups on one (launch_limits)
+    int ncu = 0, traj_per_cu = 0, pass_per_cu = 0;  // CUs; workgroups of k_traj, k_traj_pass on one (launch_limits)
     // last run
     uint64_t last_exact = 0;
     double last_host_ms = 0, last_device_ms = 0;
@@ -906,15 +907,13 @@ int qs_batch_plan(const qs_batch* b, uint32_t circuit, uint64_t seed, double noi
 
 namespace {
 
-// Trajectories of at least kWideBits qubits always run pass by pass over all
-// their tiles (k_traj_pass, one workgroup per tile of each such state) before
-// k_traj measures them: one workgroup streaming a state of 2^20 amplitudes
-// and more tile after tile is bound by its own latency.  Smaller ones do
-// where that is expected to take no longer than a workgroup each
-// (small_go_wide).  The environment variable QPP_AMD_TRAJ_WIDE_BITS sets
-// another threshold and turns the rule off (64: none).
-constexpr uint32_t kWideBits = 18;
+using qs_batch_rule::kWideBits;
 
+// Trajectories of at least kWideBits qubits run pass by pass over all their
+// tiles (k_traj_pass, one workgroup per tile of each such state) before
+// k_traj measures them, smaller ones where the rule of qs_batch_rule.hpp says
+// so.  The environment variable QPP_AMD_TRAJ_WIDE_BITS sets another threshold
+// and turns the rule off (64: none).
 bool wide_bits_set(uint32_t* bits) {
     const char* v = std::getenv("QPP_AMD_TRAJ_WIDE_BITS");
     if (!v || !*v) return false;
@@ -922,54 +921,46 @@ bool wide_bits_set(uint32_t* bits) {
     return true;
 }
 
-// Both ways in units of one workgroup's tile and pass (about 40 us of a
-// complex128 tile, launch included): pass by pass, the launches of every
-// circuit follow each other, each as many rounds of the chip's resident
-// workgroups (three per CU) as its tiles take; with a workgroup each, the
-// longest trajectory or two rounds' worth per CU.  192 trajectories of 16
-// qubits: 16.3 -> 5.7 ms (complex64 10.9 -> 3.2), 16 of them 16.1 -> 1.2 ms,
-// 3000 of 12 qubits 6.5 -> 4.7 ms; many circuits with one trajectory each
-// keep their workgroups.
-bool small_go_wide(const qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of, uint64_t ncu) {
-    std::vector<uint64_t> count(b->cls.size(), 0);
-    for (uint64_t i = 0; i < ntraj; ++i) ++count[circuit_of[i]];
-    double wide = 0, longest = 0, all = 0;
-    for (size_t c = 0; c < count.size(); ++c) {
+bool small_go_wide(const qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of) {
+    std::vector<qs_batch_rule::Circuit> cs(b->cls.size());
+    for (uint64_t i = 0; i < ntraj; ++i) ++cs[circuit_of[i]].count;
+    for (size_t c = 0; c < cs.size(); ++c) {
         const Cls& k = b->cls[c];
-        if (!count[c] || k.nb >= kWideBits) continue;
-        double launches = 0, tiles = 0;
+        cs[c].qubits = k.nb;
+        if (!cs[c].count || k.nb >= kWideBits) continue;
         for (const FPass& p : k.P.passes) {
             if (p.phase_begin >= p.phase_end || p.ntiles == 0) return false;
-            launches += double((count[c] * p.ntiles + 3 * ncu - 1) / (3 * ncu));
-            tiles += double(p.ntiles);
+            cs[c].tiles.push_back(p.ntiles);
         }
-        wide += launches;
-        longest = std::max(longest, tiles);
-        all += tiles * double(count[c]);
     }
-    return wide <= std::max(longest, all / double(2 * ncu));
+    const uint64_t ncu = uint64_t(b->ncu);
+    return qs_batch_rule::small_pass_by_pass(cs, {b->dtype == QS_C128, uint64_t(b->pass_per_cu) * ncu,
+                                                  uint64_t(b->traj_per_cu) * ncu, qs::force_exact_sampling()});
 }
 
-// b->ncu and b->traj_per_cu
+// b->ncu, b->traj_per_cu and b->pass_per_cu
 int launch_limits(qs_batch* b) {
     constexpr const char* W = "qpp_amd::batch";
     if (b->ncu) return QS_OK;
     if (int rc = qs::ensure_device()) return rc;
     const size_t shmem = (b->dtype == QS_C128 ? size_t{16} : size_t{8}) << (8 + b->reg_bits);
-    int dev = 0, ncu = 0, per_cu = 0;
+    int dev = 0, ncu = 0, traj = 0, pass = 0;
     QS_HIP(hipGetDevice(&dev), W);
     QS_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev), W);
+    auto resident = [&](auto* k, int* n) { return hipOccupancyMaxActiveBlocksPerMultiprocessor(n, k, kThreads, shmem); };
     hipError_t e;
     if (b->dtype == QS_C128)
-        e = b->reg_bits == 3
-                ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<double, 8>, kThreads, shmem)
-                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<double, 16>, kThreads, shmem);
+        e = b->reg_bits == 3 ? resident(k_traj<double, 8>, &traj) : resident(k_traj<double, 16>, &traj);
     else
-        e = b->reg_bits == 3
-                ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<float, 8>, kThreads, shmem)
-                : hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_traj<float, 16>, kThreads, shmem);
+        e = b->reg_bits == 3 ? resident(k_traj<float, 8>, &traj) : resident(k_traj<float, 16>, &traj);
     if (e != hipSuccess) return qs::fail_hip(e, W);
-    b->traj_per_cu = std::max(1, per_cu);
+    if (b->dtype == QS_C128)
+        e = b->reg_bits == 3 ? resident(k_traj_pass<double, 8>, &pass) : resident(k_traj_pass<double, 16>, &pass);
+    else
+        e = b->reg_bits == 3 ? resident(k_traj_pass<float, 8>, &pass) : resident(k_traj_pass<float, 16>, &pass);
+    if (e != hipSuccess) return qs::fail_hip(e, W);
+    b->traj_per_cu = std::max(1, traj);
+    b->pass_per_cu = std::max(1, pass);
     b->ncu = std::max(1, ncu);
     return QS_OK;
 }
@@ -983,7 +974,7 @@ uint64_t traj_grid(const qs_batch* b, uint64_t ntraj) {
 uint32_t wide_from(const qs_batch* b, uint64_t ntraj, const uint32_t* circuit_of) {
     uint32_t bits = 0;
     if (wide_bits_set(&bits)) return bits;
-    return small_go_wide(b, ntraj, circuit_of, uint64_t(b->ncu)) ? 0 : kWideBits;
+    return small_go_wide(b, ntraj, circuit_of) ? 0 : kWideBits;
 }
 
 // Bytes of states that small trajectories may hold at a time when they run

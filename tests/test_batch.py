@@ -8,6 +8,8 @@ outcome equals the oracle QNoisyEngine's for the same seed, in the
 persistent launch and on the wide path (QPP_AMD_TRAJ_WIDE_BITS sets the
 qubit count from which trajectories run pass by pass; default 18)."""
 import ctypes
+import os
+import subprocess
 
 import numpy as np
 import pytest
@@ -399,3 +401,14 @@ def test_run_states_errors():
         qa._check(run([st, st], np.zeros(2, dtype=np.uint32)))
     with pytest.raises(qa.OutOfRange):
         qa._check(run([qa.State([2] * 12)], np.ones(1, dtype=np.uint32)))
+
+
+def test_small_trajectories_rule(tmp_path):
+    """The rule that sends small trajectories pass by pass or to a workgroup
+    each (tests/cpp/batch_rule_check.cpp), for batches timed both ways: also
+    beside wide trajectories, whose exact replays hide a workgroup each."""
+    exe = str(tmp_path / "batch_rule_check")
+    src = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "batch_rule_check.cpp")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-o", exe, src], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.strip() == "ok", r.stdout
