@@ -214,7 +214,7 @@ __device__ __forceinline__ void do_scale(const cxt<R>* x, cxt<R>* y, uint32_t re
     }
 }
 
-template <typename R, int NR, int J0, int J1, bool CT>
+template <typename R, int NR, int J0, int J1, bool CT, bool SELECT>
 __device__ __forceinline__ void do_u2(const cxt<R>* x, cxt<R>* y, uint32_t regok,
                                       const cxt<R>* __restrict__ M, bool tok) {
     // column-major 4x4; gate index bit 0 <-> register bit J0, bit 1 <-> J1
@@ -236,7 +236,14 @@ __device__ __forceinline__ void do_u2(const cxt<R>* x, cxt<R>* y, uint32_t regok
         }
         cxt<R> o[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = mac4<R>(m[r], v[0], m[r + 4], v[1], m[r + 8], v[2], m[r + 12], v[3]);
+        for (int r = 0; r < 4; ++r) {
+            if constexpr (SELECT) {
+                o[r] = mac4<R>(m[r], v[0], m[r + 4], v[1], m[r + 8], v[2], m[r + 12], v[3]);
+            } else {
+                const cxt<R> s = mac2<R>(m[r], v[0], m[r + 4], v[1]), t2 = mac2<R>(m[r + 8], v[2], m[r + 12], v[3]);
+                o[r] = mk<R>(s.x + t2.x, s.y + t2.y);
+            }
+        }
         if (CT) {
             y[i0] = sel<R>(tok, o[0], v[0]);
             y[i1] = sel<R>(tok, o[1], v[1]);
@@ -280,6 +287,7 @@ __device__ __forceinline__ void run_op_ct(const cxt<R>* x, cxt<R>* y, const OpHe
                                           bool tok) {
     const uint32_t code = h.code, regok = h.regok;
     const int j0 = (code >> 4) & 3, j1 = (code >> 6) & 3;
+    if constexpr (!SELECT) __builtin_assume((code & 15u) < OP_U1S);  // (else the dispatch keeps a case for them)
     switch (code & 15u) {
         case OP_U1:
             QS_J_CASES(do_u1, x, y, regok, mu, tok)
@@ -319,19 +327,19 @@ __device__ __forceinline__ void run_op_ct(const cxt<R>* x, cxt<R>* y, const OpHe
             const cxt<R>* M = mats + h.moff;
             if (SELECT && !CT && (code & 15u) == OP_U2S && (base & op->omask) == op->oval) M += 16;
             switch (j0 * 4 + j1) {
-                case 0 * 4 + 1: do_u2<R, NR, 0, 1, CT>(x, y, regok, M, tok); break;
-                case 0 * 4 + 2: do_u2<R, NR, 0, 2, CT>(x, y, regok, M, tok); break;
-                case 1 * 4 + 2: do_u2<R, NR, 1, 2, CT>(x, y, regok, M, tok); break;
+                case 0 * 4 + 1: do_u2<R, NR, 0, 1, CT, SELECT>(x, y, regok, M, tok); break;
+                case 0 * 4 + 2: do_u2<R, NR, 0, 2, CT, SELECT>(x, y, regok, M, tok); break;
+                case 1 * 4 + 2: do_u2<R, NR, 1, 2, CT, SELECT>(x, y, regok, M, tok); break;
                 case 0 * 4 + 3:
-                    if constexpr (NR > 8) do_u2<R, NR, 0, 3, CT>(x, y, regok, M, tok);
+                    if constexpr (NR > 8) do_u2<R, NR, 0, 3, CT, SELECT>(x, y, regok, M, tok);
                     else copy_regs<R, NR>(x, y);
                     break;
                 case 1 * 4 + 3:
-                    if constexpr (NR > 8) do_u2<R, NR, 1, 3, CT>(x, y, regok, M, tok);
+                    if constexpr (NR > 8) do_u2<R, NR, 1, 3, CT, SELECT>(x, y, regok, M, tok);
                     else copy_regs<R, NR>(x, y);
                     break;
                 case 2 * 4 + 3:
-                    if constexpr (NR > 8) do_u2<R, NR, 2, 3, CT>(x, y, regok, M, tok);
+                    if constexpr (NR > 8) do_u2<R, NR, 2, 3, CT, SELECT>(x, y, regok, M, tok);
                     else copy_regs<R, NR>(x, y);
                     break;
                 default: copy_regs<R, NR>(x, y); break;
@@ -374,7 +382,10 @@ __device__ __forceinline__ OpHead load_head(const FOp* op) {
 }
 
 // y := op(x), loading the op's head here.  SELECT: pair-fused programs, with
-// OP_U1S and OP_U2S; without them the code is smaller (batches).
+// OP_U1S and OP_U2S and many 4x4s, each one FMA chain.  Without (batches, few
+// 4x4s) their cases and that chain cost k_traj_pass 3%: 1024 trajectories of
+// 16 and 128 each of 12, 20 and 22 qubits, complex128, 430 ms with both, 429
+// without the chain, 414 without either.
 template <typename R, int NR, bool SELECT = false>
 __device__ __forceinline__ void run_op(const cxt<R>* x, cxt<R>* y, const FOp* op,
                                        const double* mu, const cxt<R>* mats, uint32_t t,
