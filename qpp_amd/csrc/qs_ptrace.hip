@@ -344,6 +344,9 @@ __global__ __launch_bounds__(256) void k_ptrace(const T* __restrict__ a, T* __re
     const uint64_t rb = offset_of(keep, Ix(min(i, Dbar - 1)));
     for (uint64_t j = blockIdx.y; j < Dbar; j += gridDim.y) {
         const uint64_t cb = offset_of(keep, Ix(j));
+        // a ket's entry below the diagonal is the conjugate of the one above
+        const bool above = i <= j;
+        const uint64_t pb = above ? rb : cb, qb = above ? cb : rb;
         double sr = 0, si = 0;
         for (uint64_t t = l; t < Dsub; t += sl) {
             const uint64_t off = offset_of(tr, Ix(t));
@@ -352,7 +355,7 @@ __global__ __launch_bounds__(256) void k_ptrace(const T* __restrict__ a, T* __re
                 sr += v.x;
                 si += v.y;
             } else {
-                const T x = a[rb + off], y = a[cb + off];
+                const T x = a[pb + off], y = a[qb + off];
                 // x * conj(y)
                 const double xr = x.x, xi = x.y, yr = y.x, yi = y.y;
                 sr += xr * yr + xi * yi;
@@ -372,7 +375,7 @@ __global__ __launch_bounds__(256) void k_ptrace(const T* __restrict__ a, T* __re
         if (l == 0 && i < Dbar) {
             T v;
             v.x = sr;
-            v.y = si;
+            v.y = rho ? si : i == j ? si * 0 : above ? si : -si;  // (NaN and infinity stay NaN)
             out[i + j * Dbar] = v;
         }
     }
@@ -387,29 +390,71 @@ uint64_t count_of(const DigitList& list) {
     return c;
 }
 
-template <typename T, uint32_t W>
-int launch_gram(const qs_state* in, qs_state* out, const Digits& rows, const Digits& lo,
-                const Digits& hi, uint32_t Dbar, uint32_t grp, uint32_t TL, uint32_t nth,
-                bool rowfast) {
-    constexpr const char* where = "qpp::ptrace()";
-    const uint32_t R = Dbar * grp, nb = (R + W - 1) / W, npairs = nb * (nb + 1) / 2;
+// How the matrix products of W-row tiles are cut: slices of `per` values of
+// the outer traced index, and an estimate of the time.
+struct GramPlan {
+    uint32_t npairs, nslices, per;
+    bool whole;  // one slice of k_gram_pair writes the result itself
+    double us;
+};
+
+GramPlan gram_plan(uint32_t W, uint32_t R, uint32_t TL, uint32_t nth) {
+    const uint32_t nb = (R + W - 1) / W;
+    GramPlan g{};
+    g.npairs = nb * (nb + 1) / 2;
     // One round of resident workgroups: k_gram_pair's three per CU are 96 on
     // each XCD, which takes whole slices (one workgroup too many on an XCD is
     // a second round: 24 qubits with 8 kept, 10 pairs, take 465 us with 94
     // slices, 524 with 74, 420 with 69).  Each has at least 64 traced values
     // (below that writing the tiles shows).
-    uint32_t want = (W == 16 ? 2048 : 1024) / std::min<uint32_t>(npairs, 1024);
-    if (W == kGramW && npairs <= 96) want = 8 * (96 / npairs);
+    uint32_t want = (W == 16 ? 2048 : 1024) / std::min<uint32_t>(g.npairs, 1024);
+    if (W == kGramW && g.npairs <= 96) want = 8 * (96 / g.npairs);
     const uint32_t most = std::max<uint32_t>(1, static_cast<uint32_t>(uint64_t(TL) * nth / 64));
-    uint32_t nslices = std::min({want, most, std::max<uint32_t>(nth, 1)});
-    const uint32_t per = (nth + nslices - 1) / nslices;
-    nslices = (nth + per - 1) / per;
-    const bool direct = W == kGramW && nslices == 1;
+    g.nslices = std::min({want, most, std::max<uint32_t>(nth, 1)});
+    g.per = (nth + g.nslices - 1) / g.nslices;
+    g.nslices = (nth + g.per - 1) / g.per;
+    g.whole = W == kGramW && g.nslices == 1;
+    // a slice is serial: 0.14 us a traced value (k_gram 0.04), 81 rows of
+    // 1000 values of one digit 165 us, 30 of 3000 142
+    const double rounds = std::max(1.0, double(g.npairs) * g.nslices / 768);
+    g.us = (g.whole ? 17 : 28) + rounds * g.per * TL * (W == kGramW ? 0.14 : 0.04);
+    return g;
+}
+
+// Threads per entry of k_ptrace: as many as leave each a few terms, and more
+// where there are few entries.
+uint32_t direct_threads(uint64_t Dbar, uint64_t Dsub) {
+    uint32_t sl = 1;
+    while (sl < 256 && sl * 8 <= Dsub && Dbar * Dbar * sl < (uint64_t{1} << 18)) sl *= 2;
+    while (sl < 256 && sl < Dsub && Dbar * Dbar * sl < (uint64_t{1} << 14)) sl *= 2;
+    return sl;
+}
+
+// An estimate of k_ptrace's time on a ket.  Calls of one MI355X, either dtype
+// (matrix products / direct sums): kept 2 of 13, 14, 16 qubits 26/25, 28/42,
+// 28/158 us; 16 of 12, 16, 18 qubits 26/21, 28/26, 28/82; 64 of 12, 16, 18
+// 19/21, 29/26, 30/92; 512 of 14, 16 18/31, 35/123; 9 qutrits with 4 kept
+// 34/20, 11 with 5 40/114; one digit of 1000 kept and one traced 169/4000.
+double direct_us(uint64_t Dbar, uint64_t Dsub) {
+    const double terms = std::ceil(double(Dsub) / direct_threads(Dbar, Dsub));
+    return 19 + std::max(1.1 * (terms - 12), 2.2e-6 * double(Dbar) * double(Dbar) * double(Dsub));
+}
+
+template <typename T, uint32_t W>
+int launch_gram(const qs_state* in, qs_state* out, const Digits& rows, const Digits& lo,
+                const Digits& hi, uint32_t Dbar, uint32_t grp, uint32_t TL, uint32_t nth,
+                bool rowfast) {
+    constexpr const char* where = "qpp::ptrace()";
+    const uint32_t R = Dbar * grp;
+    const GramPlan plan = gram_plan(W, R, TL, nth);
+    const uint32_t npairs = plan.npairs, nslices = plan.nslices, per = plan.per;
+    const bool direct = plan.whole;
     double2* part = nullptr;  // at most 2048 tiles
-    if (!direct)
-        QS_HIP(hipMallocAsync(reinterpret_cast<void**>(&part),
-                              sizeof(double2) * W * W * uint64_t(npairs) * nslices, in->stream),
-               where);
+    if (!direct) {
+        const hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&part),
+                                            sizeof(double2) * W * W * uint64_t(npairs) * nslices, in->stream);
+        if (e != hipSuccess) return qs::fail_hip(e, where);
+    }
     const T* src = static_cast<const T*>(in->d);
     T* dst = static_cast<T*>(out->d);
     if constexpr (W == kGramW) {
@@ -474,17 +519,18 @@ int ptrace_impl(const qs_state* in, qs_state* out, const DigitList& keep, const 
             const auto T32 = static_cast<uint32_t>(TL), H32 = static_cast<uint32_t>(nth);
             // along the rows where the fastest kept digit is below the traced ones
             const bool rowfast = dlo.n == 0 || (drows.n && drows.str[drows.n - 1] < dlo.str[dlo.n - 1]);
-            if (Dbar * grp <= 16) return launch_gram<T, 16>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast);
-            if (Dbar <= 32) return launch_gram<T, 32>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast);
-            return launch_gram<T, kGramW>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast);
+            // the matrix products where they are expected to take less time
+            // than the direct sums (their slices cut whole digits, so one
+            // large traced digit leaves most of the chip idle)
+            const uint32_t w = Dbar * grp <= 16 ? 16 : Dbar <= 32 ? 32 : kGramW;
+            if (gram_plan(w, D32 * G32, T32, H32).us < direct_us(Dbar, Dsub))
+                return w == 16   ? launch_gram<T, 16>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast)
+                       : w == 32 ? launch_gram<T, 32>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast)
+                                 : launch_gram<T, kGramW>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast);
         }
         ts = tr;
     }
-    // threads per entry: as many as leave each a few terms, and more where
-    // there are few entries
-    uint32_t sl = 1;
-    while (sl < 256 && sl * 8 <= Dsub && Dbar * Dbar * sl < (uint64_t{1} << 18)) sl *= 2;
-    while (sl < 256 && sl < Dsub && Dbar * Dbar * sl < (uint64_t{1} << 14)) sl *= 2;
+    const uint32_t sl = direct_threads(Dbar, Dsub);
     const uint64_t gx = (Dbar + 256 / sl - 1) / (256 / sl);
     const uint64_t gy = std::min<uint64_t>(Dbar, std::max<uint64_t>(1, 16384 / gx));
     const dim3 g(static_cast<uint32_t>(gx), static_cast<uint32_t>(gy));

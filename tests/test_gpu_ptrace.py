@@ -26,6 +26,19 @@ QUDITS = [
 ]
 
 
+# large enough for the matrix products: rows at the edges of their tiles (16,
+# 32, 64 and one more), traced digits inside a slice's step and across slices,
+# rows along and across the fastest digit; and shapes on either side of the
+# rule that chooses them
+PRODUCTS = [
+    ([16] + [2] * 13, list(range(1, 14))), ([2] * 13 + [16], list(range(13))), ([17, 2, 4, 8, 4, 8, 4], [1, 2, 3, 4, 5, 6]),
+    ([32] + [2] * 13, list(range(1, 14))), ([2] * 12 + [33], list(range(12))), ([8, 3, 8, 5, 8, 3, 9], [1, 3, 4, 5, 6]),
+    ([64] + [2] * 11, list(range(1, 12))), ([2] * 11 + [65], list(range(11))), ([3] * 11, [0, 1, 3, 5, 7, 10]),
+    ([129, 5, 3, 7, 4], [1, 2, 3, 4]), ([4, 31, 9, 31], [0, 2]), ([81, 1000], [1]), ([1000, 30], [0]), ([17, 4000], [1]),
+    ([3] * 9, [4, 5, 6, 7, 8]), ([50, 20, 100], [1, 2]), ([40, 4096], [1]), ([500, 600], [0]),
+]
+
+
 def _check(qa, orc, dims, traced, dtype, rng):
     psi = randket(int(np.prod(dims)), rng)
     if dtype == "c64":
@@ -48,6 +61,13 @@ def test_ptrace_ket_qubits(qa, orc, n, traced, dtype):
 @pytest.mark.parametrize("dims,traced", QUDITS)
 def test_ptrace_ket_qudits(qa, orc, dims, traced, dtype):
     _check(qa, orc, dims, traced, dtype, np.random.default_rng(len(dims)))
+
+
+@pytest.mark.parametrize("dtype", ["c128", "c64"])
+@pytest.mark.parametrize("dims,traced", PRODUCTS)
+def test_ptrace_ket_products(qa, orc, dims, traced, dtype):
+    got = _check(qa, orc, dims, traced, dtype, np.random.default_rng(len(dims) + dims[0]))
+    assert np.array_equal(got, got.conj().T)  # either way one triangle is the other's conjugate
 
 
 @pytest.mark.parametrize("dims,traced", [([2] * 9, [0]), ([2] * 9, [8]), ([2] * 9, list(range(1, 9))), ([2] * 9, [2, 5, 0]),
