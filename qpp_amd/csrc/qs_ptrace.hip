@@ -440,6 +440,9 @@ double direct_us(uint64_t Dbar, uint64_t Dsub) {
     return 19 + std::max(1.1 * (terms - 12), 2.2e-6 * double(Dbar) * double(Dbar) * double(Dsub));
 }
 
+// launch_gram: no memory for the partial tiles
+constexpr int kNoRoom = -1;
+
 template <typename T, uint32_t W>
 int launch_gram(const qs_state* in, qs_state* out, const Digits& rows, const Digits& lo,
                 const Digits& hi, uint32_t Dbar, uint32_t grp, uint32_t TL, uint32_t nth,
@@ -453,6 +456,10 @@ int launch_gram(const qs_state* in, qs_state* out, const Digits& rows, const Dig
     if (!direct) {
         const hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&part),
                                             sizeof(double2) * W * W * uint64_t(npairs) * nslices, in->stream);
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();  // handled: not the next call's
+            return kNoRoom;
+        }
         if (e != hipSuccess) return qs::fail_hip(e, where);
     }
     const T* src = static_cast<const T*>(in->d);
@@ -523,10 +530,12 @@ int ptrace_impl(const qs_state* in, qs_state* out, const DigitList& keep, const 
             // than the direct sums (their slices cut whole digits, so one
             // large traced digit leaves most of the chip idle)
             const uint32_t w = Dbar * grp <= 16 ? 16 : Dbar <= 32 ? 32 : kGramW;
+            int rc = kNoRoom;
             if (gram_plan(w, D32 * G32, T32, H32).us < direct_us(Dbar, Dsub))
-                return w == 16   ? launch_gram<T, 16>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast)
-                       : w == 32 ? launch_gram<T, 32>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast)
-                                 : launch_gram<T, kGramW>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast);
+                rc = w == 16   ? launch_gram<T, 16>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast)
+                     : w == 32 ? launch_gram<T, 32>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast)
+                               : launch_gram<T, kGramW>(in, out, drows, dlo, dhi, D32, G32, T32, H32, rowfast);
+            if (rc != kNoRoom) return rc;
         }
         ts = tr;
     }
