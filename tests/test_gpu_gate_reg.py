@@ -77,6 +77,24 @@ def test_rho_gates(qa, orc, n, dtype):
             assert np.max(np.abs(st.apply_kraus(Ks, t).download() - orc.apply_kraus(rho, Ks, t, 2))) <= tol, t
 
 
+@pytest.mark.parametrize("n,k,ctrl,dtype", [(11, 1, [0, 1], "c128"), (11, 1, [1, 0, 10], "c128"),
+                                            (11, 1, [0, 10], "c128"), (12, 1, [2, 0], "c64"),
+                                            (12, 2, [5, 0, 1], "c64"), (12, 2, [0, 11], "c64")])
+def test_rho_gates_under_many_controls(qa, orc, n, k, ctrl, dtype):
+    """Density matrices large enough that two and more controls above the
+    lane bits take rows and columns in a pass each, and neighbours that do
+    not."""
+    rng = np.random.default_rng(n + len(ctrl))
+    dt, tol = _dt(qa, dtype)
+    D = 2 ** n
+    rho = (rng.standard_normal((D, D)) + 1j * rng.standard_normal((D, D))) / D
+    U, t, sh = _haar(2 ** k, rng), [6, 3][:k], [int(x) for x in rng.integers(0, 2, len(ctrl))]
+    print(f"rho n={n} k={k} controls {ctrl} {dtype}", flush=True)
+    st = qa.State.from_array(rho, [2] * n, dtype=dt)
+    got = st.apply_ctrl(U, ctrl, t, sh).download()
+    assert np.max(np.abs(got - orc.applyCTRL(rho, U, ctrl, t, 2, sh))) <= tol
+
+
 @pytest.mark.parametrize("k", [4, 5])
 def test_gates_from_two_threads(qa, k):
     """Commuting (diagonal) gates applied to one state by two threads at once,
