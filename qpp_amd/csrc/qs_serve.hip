@@ -123,9 +123,10 @@ bool batchable(const qs_circuit* c) {
 //   post-selection retries: the saved state and the first
 //   successful rep's state (execute_with_retries)           2 s D
 //   a destructive measurement's contracted output           s D / 2
-//   the sampler's workspace: FP64 probabilities and the
-//   exact cumulative table (2 x 8 D), block tables and
-//   per-shot slots (qs_measure.hip)                         16 D + 64 D / 4096 + 24 shots
+//   the sampler's workspace: FP64 probabilities (8 D; the
+//   exact cumulative table takes their place), block
+//   tables and per-shot slots (qs_measure.hip), and 8 D of
+//   room that callers' budgets have always counted           16 D + 64 D / 4096 + 24 shots
 // plus 2 MiB for the compiled passes' tables and small buffers.  The
 // sampling-tail path holds less (the state, its pre-measurement copy and the
 // workspace), so this bound covers it.

@@ -53,6 +53,30 @@ def test_rho(qa, orc, n, destructive):
         assert np.max(np.abs(st.download().reshape(-1) - np.asarray(left).reshape(-1))) <= 1e-12, (t, u)
 
 
+@pytest.mark.parametrize("destructive", [False, True])
+@pytest.mark.parametrize("n,dtype", [(4, "c64"), (6, "c64"), (10, "c128"), (11, "c128"), (11, "c64")])
+def test_rho_more(qa, orc, n, dtype, destructive):
+    """complex64 density matrices, and those of more than 10 subsystems,
+    which are projected from the last target down when destructive
+    (instruments.hpp:1055-1095): each probability is conditioned on the
+    targets before it in that order."""
+    rng = np.random.default_rng(100 + n)
+    dt, tol = (qa.C128, 1e-12) if dtype == "c128" else (qa.C64, 2e-6)
+    D = 2 ** n
+    vs = [randket(D, rng) for _ in range(2)]
+    rho = sum(w * np.outer(v, v.conj()) for w, v in zip((0.6, 0.4), vs))
+    if dtype == "c64":
+        rho = rho.astype(np.complex64).astype(np.complex128)
+    for t in ([2, 0, n - 1], [n - 1, 1], [1]):
+        u = float(rng.random())
+        print(f"rho n={n} {dtype} targets {t} destructive={destructive}", flush=True)
+        st = qa.State.from_array(rho, [2] * n, dtype=dt)
+        res, ps = st.measure_seq(t, u, destructive)
+        r, p, left = orc.measure_seq(rho, t, 2, destructive, u)
+        assert list(r) == res and np.max(np.abs(np.array(ps) - p)) <= tol, (t, u)
+        assert np.max(np.abs(st.download().reshape(-1) - np.asarray(left).reshape(-1))) <= tol, (t, u)
+
+
 def test_impossible_result(qa):
     """u = 0 selects index 0 also where its probability is 0; dividing by the
     weight 0 leaves no number behind, as target by target."""

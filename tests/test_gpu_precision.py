@@ -119,8 +119,8 @@ def _dense_cases(n, rng):
 @pytest.mark.parametrize("valu", [False, True])
 def test_c64_dense_gates_mfma_vs_oracle(orc, monkeypatch, valu):
     """4- and 5-qubit dense gates on complex64 kets and density matrices
-    (FP32 MFMA kernel; valu: the VALU kernel forced by QPP_AMD_GATEK_VALU)
-    against the complex128 oracle: max-abs <= 2e-6 (FP32 sums of up to 32
+    (registers and FP32 MFMA kernel; valu: the kernel for any width forced by
+    QPP_AMD_GATEK_VALU) against the complex128 oracle: max-abs <= 2e-6 (FP32 sums of up to 32
     terms of a unit column)."""
     if valu:
         monkeypatch.setenv("QPP_AMD_GATEK_VALU", "1")
