@@ -250,8 +250,9 @@ def bench_batch(args, qa):
         "outcomes_equal_c128_batch": agree,
         "oracle_outcomes_matched": f"{om}/{len(i12)} (12-qubit), {om16}/{len(i16)} (16-qubit)",
         "roofline": {"bound": "hbm",
-                     "kernel": "k_traj_pass (20- and 22-qubit members, pass by pass, a workgroup per "
-                               "tile) + k_traj (persistent: 12- and 16-qubit members, every measurement)",
+                     "kernel": "k_traj_pass (20- and 22-qubit members, small ones too where the batch's "
+                               "rule says so, pass by pass, a workgroup per "
+                               "tile) + k_traj (persistent: the others, every measurement)",
                      "achieved": round(achieved, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,

@@ -580,7 +580,10 @@ __global__ __launch_bounds__(kBlock) void k_qudit(cxt<R>* __restrict__ a,
 // each).  cshift[k] is digit k's control shift, or -1 for a spectator that
 // controls nothing.  Threads of a wave with different powers of A take them
 // in turn, so that the matrix is always uniform (scalar loads).  14 qutrits
-// complex128: 100 -> 27 us a gate on one, 48 on two; HBM bounds it.
+// complex128: 100 -> 27 us a gate on one, 48 on two; HBM bounds it.  Wider
+// gates, on two qudits of different dimensions or three of any, stay with
+// k_qudit: a group of 27 and more complex128 amplitudes leaves few waves to a
+// SIMD, and those widths have not been measured here.
 struct QGFast {
     Digits sp;
     int32_t cshift[kMaxDigits];

@@ -35,7 +35,8 @@ PRODUCTS = [
     ([32] + [2] * 13, list(range(1, 14))), ([2] * 12 + [33], list(range(12))), ([8, 3, 8, 5, 8, 3, 9], [1, 3, 4, 5, 6]),
     ([64] + [2] * 11, list(range(1, 12))), ([2] * 11 + [65], list(range(11))), ([3] * 11, [0, 1, 3, 5, 7, 10]),
     ([129, 5, 3, 7, 4], [1, 2, 3, 4]), ([4, 31, 9, 31], [0, 2]), ([81, 1000], [1]), ([1000, 30], [0]), ([17, 4000], [1]),
-    ([3] * 9, [4, 5, 6, 7, 8]), ([50, 20, 100], [1, 2]), ([40, 4096], [1]), ([500, 600], [0]),
+    ([3] * 9, [4, 5, 6, 7, 8]), ([50, 20, 100], [1, 2]), ([40, 4096], [1]), ([300, 4096], [1]),
+    ([500, 600], [0]),
 ]
 
 
